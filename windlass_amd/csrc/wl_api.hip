@@ -927,11 +927,33 @@ static int moe_check(const wl_weight *g, const wl_weight *u, const wl_weight *d,
   return WL_OK;
 }
 
+// each: passes of 8 tokens whatever T is, so that a token's bits do not depend on the batch
+// (ForwardBatch's rows; the host entry, which counts each pass's experts).
 static int moe_dev(wl_ctx *c, const float *d_logits, int32_t k, int32_t renorm, const wl_weight *g,
-                   const wl_weight *u, const wl_weight *d, const float *d_x, int32_t T, float *d_out) {
+                   const wl_weight *u, const wl_weight *d, const float *d_x, int32_t T, float *d_out, bool each) {
   int rc = moe_check(g, u, d, k);
   if (rc) return rc;
   const int ne = g->experts, ff = (int)g->rows, embd = (int)g->cols;
+  if (!each && !c->int_dot && wl::moe_many_applies(g->type, d->type, T, ne, ff, embd)) {
+    // a prompt: every chosen expert's weights once per MOE_MANY_T tokens; the passes share the
+    // tokens evenly (each more than 8)
+    const int passes = (T + wl::MOE_MANY_T - 1) / wl::MOE_MANY_T, per = (T + passes - 1) / passes;
+    if ((rc = ensure(c, S_MOE, (size_t)wl::moe_many_scratch_bytes(per, k, ne, ff, embd)))) return rc;
+    for (int t0 = 0; t0 < T; t0 += per) {
+      wl::MoeLaunch m{};
+      m.logits = d_logits + (int64_t)t0 * ne;
+      m.T = T - t0 < per ? T - t0 : per;
+      m.ne = ne; m.k = k; m.renorm = renorm;
+      m.gu_type = g->type; m.d_type = d->type;
+      m.gate = g->dev; m.up = u->dev; m.down = d->dev;
+      m.gu_row_bytes = g->row_bytes; m.d_row_bytes = d->row_bytes;
+      m.ff = ff; m.embd = embd;
+      m.x = d_x + (int64_t)t0 * embd;
+      m.out = d_out + (int64_t)t0 * embd;
+      WL_HIP(wl::moe_many_launch(m, c->buf[S_MOE], c->stream), "moe launch");
+    }
+    return WL_OK;
+  }
   if (!c->buf[S_MSYNC]) {
     if ((rc = ensure(c, S_MSYNC, sizeof(wl::MoeSync)))) return rc;
     WL_HIP(wl::moe_sync_init((wl::MoeSync *)c->buf[S_MSYNC], c->stream), "moe counters");
@@ -979,7 +1001,7 @@ extern "C" int wl_moe_ffn_dev(wl_ctx *c, const float *d_logits, int32_t k, int32
                               const wl_weight *u, const wl_weight *d, const float *d_x, int32_t T, float *d_out) {
   if (!c || !d_logits || !d_x || !d_out) return fail(WL_E_ARG, "wl_moe_ffn_dev: null argument");
   if (T <= 0) return fail(WL_E_SHAPE, "MatMul shape mismatch: T = %d", T);
-  return moe_dev(c, d_logits, k, renorm, g, u, d, d_x, T, d_out);
+  return moe_dev(c, d_logits, k, renorm, g, u, d, d_x, T, d_out, false);
 }
 
 extern "C" int wl_moe_ffn(wl_ctx *c, const float *logits, int32_t k, int32_t renorm, const wl_weight *g,
@@ -998,7 +1020,7 @@ extern "C" int wl_moe_ffn(wl_ctx *c, const float *logits, int32_t k, int32_t ren
   for (int t0 = 0; t0 < T; t0 += wl::MOE_MAX_T) {
     const int Tc = T - t0 < wl::MOE_MAX_T ? T - t0 : wl::MOE_MAX_T;
     if ((rc = moe_dev(c, (const float *)c->buf[S_AUX] + (int64_t)t0 * ne, k, renorm, g, u, d,
-                      (const float *)c->buf[S_X] + (int64_t)t0 * embd, Tc, (float *)c->buf[S_OUT] + (int64_t)t0 * embd)))
+                      (const float *)c->buf[S_X] + (int64_t)t0 * embd, Tc, (float *)c->buf[S_OUT] + (int64_t)t0 * embd, true)))
       return rc;
     if (expert_runs) {
       MoeScratch s = moe_layout(Tc, k, ne, (int)g->rows, embd);
@@ -1392,7 +1414,8 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
     return rc;
   float *lg = (float *)c->buf[S_LR], *o = (float *)c->buf[S_LM], *sh = (float *)c->buf[S_LS];
   if ((rc = mm(L->ffn_gate_inp, fin, lg, false))) return rc;
-  if ((rc = moe_dev(c, lg, L->expert_used, L->expert_weights_norm, L->ffn_gate, L->ffn_up, L->ffn_down, fin, T, o)))
+  if ((rc = moe_dev(c, lg, L->expert_used, L->expert_weights_norm, L->ffn_gate, L->ffn_up, L->ffn_down, fin, T, o,
+                    each)))
     return rc;
   if (shared) {
     if ((rc = swiglu(L->ffn_gate_shexp, L->ffn_up_shexp, L->ffn_down_shexp, sh, false))) return rc;

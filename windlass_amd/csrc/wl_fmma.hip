@@ -23,41 +23,18 @@
 // quarter q of each super-block and feeds the MFMA's B operand; the A operand (16 columns of x
 // parts) comes from LDS, one 16-byte read per MFMA, conflict-free.
 #include "wl_fmma.h"
+#include "wl_fmma_codec.h"
 #include "wl_gemv_launch.h"
 
 #pragma clang fp contract(off)
 
 namespace wl {
 
-typedef _Float16 fh2 __attribute__((ext_vector_type(2)));
-typedef _Float16 fh4 __attribute__((ext_vector_type(4)));
-typedef _Float16 fh8 __attribute__((ext_vector_type(8)));
-typedef float ff4 __attribute__((ext_vector_type(4)));
-
 constexpr int FM_UNIT = 2048;                        // columns per unit: 8 super-blocks
 constexpr int FM_NS = 16;                            // MFMA columns (two per token)
 constexpr int FM_XBYTES = 8 * 8 * 4 * FM_NS * 16;    // x parts: [sb][m][q][slot] of 8 halves
 constexpr int FM_SBYTES = 8 * 2 * 4 * FM_NS * 4;     // Q4_K sub-block sums: [sb][half][q][slot]
 constexpr int FM_WAVES = 8;
-
-__device__ __forceinline__ fh2 as_fh2(uint32_t u) { return __builtin_bit_cast(fh2, u); }
-__device__ __forceinline__ uint32_t as_u32(fh2 v) { return __builtin_bit_cast(uint32_t, v); }
-
-// The unit's scale: f = 2^(15 - e) for the largest finite |x| = m 2^e (m in [0.5, 1)), and 1/f;
-// both powers of two, clamped to the normal range. An all-zero (or non-finite) unit takes f = 1.
-__device__ __forceinline__ void unit_scale(float mx, float &f, float &inv) {
-  if (!(mx > 0.f)) {
-    f = 1.f;
-    inv = 1.f;
-    return;
-  }
-  int e;
-  frexpf(mx, &e);
-  int s = 15 - e;
-  s = s > 126 ? 126 : s;
-  f = ldexpf(1.f, s);
-  inv = ldexpf(1.f, -s);
-}
 
 // One token's parts of one unit, by one wave: lane (sb = l / 8, e = l % 8) reads 32 values,
 // the wave takes the largest finite |x|, and the lane writes its values' hi and lo halves to

@@ -42,6 +42,19 @@ struct MoeSync {
   unsigned err[MOE_SYNC_LINE];
 };
 
+// The plan of a pass of many tokens (wl_moe_mma.hip), on the device: tiles of pairs of one
+// expert, the pairs' tokens, and each token's pairs in ascending expert order with their weights.
+struct MoeTile {
+  int expert, first, n;
+};
+struct MoeMany {
+  int *ntiles;
+  MoeTile *tiles;
+  int *pair_tok;   // [pairs]
+  int *comb_pair;  // [T][k]
+  float *comb_w;   // [T][k]
+};
+
 struct MoeGemvArgs {
   const MoePlan *plan;
   const uint8_t *w, *w2;
@@ -91,6 +104,13 @@ hipError_t route_launch(const float *logits, int T, int n, int k, int renorm, in
 // the other set for the next one-launch launch), rather than the launch chain.
 bool moe_uses_one_launch(const MoeLaunch &m);
 hipError_t moe_launch(const MoeLaunch &m, int num_cu, hipStream_t st);
+// MoeFfn of more than MOE_MAX_T tokens at once on the matrix cores, each chosen expert's weights
+// read once (wl_moe_mma.hip): whether it takes these experts, its scratch and its launches (l's
+// own scratch pointers are not used). Tokens per pass at most MOE_MANY_T, which bounds the scratch.
+constexpr int MOE_MANY_T = 1024;
+bool moe_many_applies(int gu_type, int d_type, int T, int ne, int ff, int embd);
+int64_t moe_many_scratch_bytes(int T, int k, int ne, int ff, int embd);
+hipError_t moe_many_launch(const MoeLaunch &l, void *scratch, hipStream_t st);
 // Zeroes a MoeSync once after its allocation (a kernel, so it may sit in a captured stream).
 hipError_t moe_sync_init(MoeSync *s, hipStream_t st);
 
