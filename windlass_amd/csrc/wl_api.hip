@@ -1135,7 +1135,7 @@ extern "C" int wl_attention_dev(wl_ctx *c, const float *d_q, int32_t T, int32_t 
     return fail(WL_E_SHAPE, "wl_attention_dev: %d heads over %d KV heads", heads, kv_heads);
   const int kv_dim = kv_heads * head_dim;
   int rc = ensure(c, S_ATT,
-                  (size_t)wl::attention_scratch_floats(T, heads, head_dim, kv_dim, pos0 + T, d_K, d_V) * sizeof(float));
+                  (size_t)wl::attention_scratch_floats(T, heads, head_dim, kv_dim, pos0 + T, d_K, d_V, wl::RowMap{}) * sizeof(float));
   if (rc) return rc;
   const int64_t qd = (int64_t)heads * head_dim;
   WL_HIP(wl::attention_launch(d_q, qd, T, d_K, d_V, kv_heads * head_dim, heads, kv_heads, head_dim, pos0, scale,
@@ -1315,7 +1315,7 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
       (rc = ensure(c, S_LK, (size_t)T * KD * 4)) || (rc = ensure(c, S_LV, (size_t)T * KD * 4)) ||
       (rc = ensure(c, S_LATT, (size_t)T * QD * 4)) ||
       (rc = ensure(c, S_LG, (size_t)T * FF * 4)) || (rc = ensure(c, S_LU, (size_t)T * FF * 4)) ||
-      (rc = ensure(c, S_ATT, (size_t)wl::attention_scratch_floats(T, H, HD, KD, max_n, d_K, d_V) * 4)))
+      (rc = ensure(c, S_ATT, (size_t)wl::attention_scratch_floats(T, H, HD, KD, max_n, d_K, d_V, rm) * 4)))
     return rc;
   float *xn = (float *)c->buf[S_LXN], *q = (float *)c->buf[S_LQ], *k = (float *)c->buf[S_LK],
         *v = (float *)c->buf[S_LV], *att = (float *)c->buf[S_LATT],

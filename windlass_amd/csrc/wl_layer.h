@@ -27,7 +27,7 @@ hipError_t kv_store_launch(const float *k, const float *v, int64_t n, uint16_t *
 // Floats of scratch attention_launch needs for these operands; max_n: the most positions a row
 // attends to (pos0 + T for one sequence).
 int64_t attention_scratch_floats(int T, int heads, int hd, int kv_dim, int max_n, const uint16_t *K,
-                                 const uint16_t *V);
+                                 const uint16_t *V, const RowMap &rm);
 hipError_t attention_launch(const float *q, int64_t ldq, int T, const uint16_t *K, const uint16_t *V, int kv_dim,
                             int heads, int kv_heads, int hd, int pos0, float scale, float *scratch, float *out,
                             int64_t ldo, const RowMap &rm, int max_n, hipStream_t st);

@@ -9,6 +9,7 @@
 // of a head adds its positions in order, RoPE's angles come from the same running product in
 // double. The double sums the reference runs sequentially (RMSNorm's sum of squares, the
 // softmax denominator) are tree sums here, so their last bit can differ.
+#include "wl_attention.h"
 #include "wl_layer.h"
 
 #include "wl_device.h"
@@ -586,8 +587,8 @@ __device__ __forceinline__ void wave_attend(const uint4 *__restrict__ ks4, const
   }
 }
 
-// Attention for the rows of a prompt (T consecutive positions pos0.. of one sequence, head dims 64
-// and 128): one workgroup of RW waves per (query head, chunk of kAttP positions, RW rows), the
+// Attention for a prompt of 2 to 15 rows (T consecutive positions pos0.. of one sequence, head dims 64
+// and 128; more rows take the matrix cores, wl_attention.hip): one workgroup of RW waves per (query head, chunk of kAttP positions, RW rows), the
 // chunk's keys (rows padded to HD + 8 halves, so sixteen lanes reading sixteen rows hit every
 // bank once) and values staged in LDS once for the RW rows, wave w computing row w of the tile
 // with wave-wide reductions and no workgroup barrier after the staging. (One workgroup per row
@@ -924,11 +925,13 @@ static bool attention_chunked(int hd, int kv_dim, const uint16_t *K, const uint1
 }
 
 int64_t attention_scratch_floats(int T, int heads, int hd, int kv_dim, int max_n, const uint16_t *K,
-                                 const uint16_t *V) {
+                                 const uint16_t *V, const RowMap &rm) {
   if (T <= 0) return 0;
   if (!attention_chunked(hd, kv_dim, K, V)) return (int64_t)T * heads * max_n;
   const int chunks = (max_n + kAttP - 1) / kAttP;
-  return chunks > 1 ? (int64_t)T * heads * chunks * (hd + 4) : 0;
+  const int64_t rows = chunks > 1 ? (int64_t)T * heads * chunks * (hd + 4) : 0;
+  if (rm.pos || !attention_tiles_applies(T, hd)) return rows;
+  return attention_tiles_scratch_floats(T, heads, kv_dim / hd, hd, max_n);
 }
 
 template <int HD, bool ROPE>
@@ -970,6 +973,8 @@ hipError_t attention_launch(const float *q, int64_t ldq, int T, const uint16_t *
                             int heads, int kv_heads, int hd, int pos0, float scale, float *scratch, float *out,
                             int64_t ldo, const RowMap &rm, int max_n, hipStream_t st) {
   if (T <= 0) return hipSuccess;
+  if (!rm.pos && !rm.slot && attention_tiles_applies(T, hd) && attention_chunked(hd, kv_dim, K, V))
+    return attention_tiles_launch(q, ldq, T, K, V, kv_dim, heads, kv_heads, hd, pos0, scale, scratch, out, ldo, st);
   if (T > 1 && !rm.pos && !rm.slot && attention_chunked(hd, kv_dim, K, V)) {  // a prompt's rows
     const int chunks = (max_n + kAttP - 1) / kAttP;
     constexpr int RW = WL_ATT_ROWS;
