@@ -18,6 +18,7 @@
 #include "wl_dequant.h"
 #include "wl_fmma.h"
 #include "wl_gemm.h"
+#include "wl_gemm_short.h"
 #include "wl_gemv.h"
 #include "wl_intdot.h"
 #include "wl_layer.h"
@@ -637,6 +638,27 @@ static int intdot_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int
   return int_run(c, w, base, nullptr, rows, d_x, acts, T, d_y, fixed);
 }
 
+// A prompt of 9 to 128 tokens (wl_gemm_short.h): x as pieces, then the products, added into d_y
+// times rs with add.
+static size_t short_bytes(const wl_weight *w, int T) {
+  return (size_t)wl::frag_bytes(T, (int)w->cols, wl::short_order(w->type));
+}
+
+static wl::ShortMat short_mat(const wl_weight *w, float *d_y) {
+  return wl::ShortMat{w->dev, w->row_bytes, (int)w->rows, w->type, d_y, w->rows};
+}
+
+static int short_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int64_t rows, const float *d_x, int T,
+                        float *d_y, bool add, float rs, void *fixed) {
+  const int cols = (int)w->cols;
+  void *xf = nullptr;
+  if (int rc = scratch_for(c, S_XB, short_bytes(w, T), fixed, &xf)) return rc;
+  WL_HIP(wl::short_frag_launch(d_x, T, cols, wl::short_order(w->type), xf, c->stream), "gemm operands");
+  const wl::ShortMat m{base, w->row_bytes, (int)rows, w->type, d_y, rows};
+  WL_HIP(wl::short_matmul_launch(&m, 1, cols, xf, T, add, rs, c->num_cu, c->stream), "gemm launch");
+  return WL_OK;
+}
+
 // fixed: the static scratch (the allocation-free entry point), or null for the context's slots.
 static int matmul_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float *d_x, int32_t T, float *d_y,
                       void *fixed = nullptr) {
@@ -650,6 +672,8 @@ static int matmul_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float
   int64_t rows;
   operand(w, expert, &base, &rows);
   if (int_path(c, w)) return intdot_matmul(c, w, base, rows, d_x, T, d_y, fixed);
+  if (wl::short_applies(w->type, T, w->cols) && (!fixed || short_bytes(w, T) <= kStaticScratchBytes))
+    return short_matmul(c, w, base, rows, d_x, T, d_y, false, 0.f, fixed);
   if (T > 8 && wl::gemm_supports(w->type)) {
     void *xb = nullptr;
     if ((rc = scratch_for(c, S_XB, (size_t)wl::gemm_scratch_bytes(w->type, (int)rows, (int)w->cols, T, c->num_cu), fixed,
@@ -687,7 +711,7 @@ extern "C" int wl_matmul_dev_noalloc(wl_ctx *c, const wl_weight *w, int32_t expe
   return matmul_dev(c, w, expert, d_x, T, d_y, fixed);
 }
 
-// d_y += (W x) * rs. Up to 8 tokens on the GEMV kernels the add is their final store; otherwise
+// d_y += (W x) * rs. Up to 128 tokens on the float kernels the add is their final store; otherwise
 // the product goes to scratch and the residual kernel adds it. Either way o = W x is rounded to
 // float first, then x + o * rs as two roundings (src/Transformer.cs:224,231).
 extern "C" int wl_matmul_add_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float *d_x, int32_t T,
@@ -705,6 +729,8 @@ extern "C" int wl_matmul_add_dev(wl_ctx *c, const wl_weight *w, int32_t expert, 
     m.rs = rs;
     return gemv(c, &m, 1, 1, d_x, (int)w->cols, T);
   }
+  if (wl::short_applies(w->type, T, w->cols) && !int_path(c, w))
+    return short_matmul(c, w, base, rows, d_x, T, d_y, true, rs, nullptr);
   if ((rc = ensure(c, S_LO, (size_t)T * rows * sizeof(float)))) return rc;
   float *o = (float *)c->buf[S_LO];
   if ((rc = matmul_dev(c, w, expert, d_x, T, o))) return rc;
@@ -1333,15 +1359,42 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
     }
     return WL_OK;
   };
+  // Prompts of 9 to 128 tokens whose matrices read x in one order: the norm writes x as pieces, the
+  // matrices that share x are one launch, and gate and up write the down product's pieces.
+  auto one_order = [&](const wl_weight *const *ws, int n) {
+    for (int i = 0; i < n; i++)
+      if (each || !wl::short_applies(ws[i]->type, T, ws[i]->cols) || int_path(c, ws[i]) || ws[i]->experts != 1 ||
+          wl::short_order(ws[i]->type) != wl::short_order(ws[0]->type))
+        return false;
+    return true;
+  };
+  auto pieces = [&](const float *norm, int ord, void **xf) -> int {
+    if (int r = ensure(c, S_XB, (size_t)wl::frag_bytes(T, E, ord))) return r;
+    *xf = c->buf[S_XB];
+    if (norm && wl::rms_norm_frag_applies(d_x, E, norm)) {
+      WL_HIP(wl::rms_norm_frag_launch(d_x, T, E, norm, L->eps, ord, *xf, c->stream), "rms norm");
+      return WL_OK;
+    }
+    if (norm)
+      if (int r = wl_rms_norm_dev(c, d_x, T, E, norm, L->eps, xn)) return r;
+    WL_HIP(wl::short_frag_launch(norm ? xn : d_x, T, E, ord, *xf, c->stream), "gemm operands");
+    return WL_OK;
+  };
   // attention block (x itself is the input under post-norms: OLMo 2 has no pre-norm)
   const float *ain = post ? d_x : xn;
-  if (!post && (rc = wl_rms_norm_dev(c, d_x, T, E, L->d_attn_norm, L->eps, xn))) return rc;
-  if (T <= 8 || each) {
+  const wl_weight *qkv[3] = {L->attn_q, L->attn_k, L->attn_v};
+  const bool qkv_one = one_order(qkv, 3);
+  if (!post && !qkv_one && (rc = wl_rms_norm_dev(c, d_x, T, E, L->d_attn_norm, L->eps, xn))) return rc;
+  if (qkv_one) {
+    void *xf;
+    if ((rc = pieces(post ? nullptr : L->d_attn_norm, wl::short_order(L->attn_q->type), &xf))) return rc;
+    const wl::ShortMat m[3] = {short_mat(L->attn_q, q), short_mat(L->attn_k, k), short_mat(L->attn_v, v)};
+    WL_HIP(wl::short_matmul_launch(m, 3, E, xf, T, false, 0.f, c->num_cu, c->stream), "q, k, v");
+  } else if (T <= 8 || each) {
     for (int t0 = 0; t0 < T; t0 += 8) {  // q, k, v in one launch per 8 rows
       const int n = T - t0 < 8 ? T - t0 : 8;
-      const wl_weight *ws[3] = {L->attn_q, L->attn_k, L->attn_v};
       float *ys[3] = {q + (int64_t)t0 * QD, k + (int64_t)t0 * KD, v + (int64_t)t0 * KD};
-      if ((rc = wl_matmul_multi_dev(c, 3, ws, ain + (int64_t)t0 * E, n, ys))) return rc;
+      if ((rc = wl_matmul_multi_dev(c, 3, qkv, ain + (int64_t)t0 * E, n, ys))) return rc;
     }
   } else if ((rc = mm(L->attn_q, ain, q, false)) || (rc = mm(L->attn_k, ain, k, false)) ||
              (rc = mm(L->attn_v, ain, v, false))) {
@@ -1380,6 +1433,18 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
   }
   // feed-forward block
   const float *fin = post ? d_x : xn;
+  const wl_weight *gu[2] = {L->ffn_gate, L->ffn_up};
+  if (!moe && !post && L->ffn_gate->type == L->ffn_up->type && one_order(gu, 2) && one_order(&L->ffn_down, 1)) {
+    void *xf;
+    if ((rc = pieces(L->d_ffn_norm, wl::short_order(L->ffn_gate->type), &xf))) return rc;
+    // the pieces of h (2 bytes a value, tokens rounded up to 16) fit T > 8 rows of floats
+    WL_HIP(wl::short_swiglu_launch(short_mat(L->ffn_gate, nullptr), short_mat(L->ffn_up, nullptr), E, xf, T, g,
+                                   wl::short_order(L->ffn_down->type), c->stream),
+           "gate and up");
+    const wl::ShortMat m = short_mat(L->ffn_down, d_x);
+    WL_HIP(wl::short_matmul_launch(&m, 1, (int)FF, g, T, true, rs, c->num_cu, c->stream), "down");
+    return WL_OK;
+  }
   if (!post && (rc = wl_rms_norm_dev(c, d_x, T, E, L->d_ffn_norm, L->eps, xn))) return rc;
   // SwiGlu (src/Transformer.cs:241-251) into y (added into y with add): up to 8 rows (or every
   // row with each) gate and up in one GEMV launch with the SiLU epilogue; a prompt: the two

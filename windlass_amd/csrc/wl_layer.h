@@ -15,6 +15,11 @@ struct RowMap {
 
 hipError_t rms_norm_launch(const float *x, int64_t rows, int64_t dim, const float *w, float eps, float *y,
                            hipStream_t st);
+// The same rows as bf16 pieces in order ord of wl_frag.h, where they apply: rows of whole 256-value
+// blocks, 16-byte aligned.
+bool rms_norm_frag_applies(const float *x, int64_t dim, const float *w);
+hipError_t rms_norm_frag_launch(const float *x, int rows, int64_t dim, const float *w, float eps, int ord, void *xf,
+                                hipStream_t st);
 // RoPE on T rows of `heads` heads (row t at pos[t], or pos0 + t when pos is null).
 hipError_t rope_launch(float *x, int64_t ldx, int T, int heads, int hd, int n, int neox, const int *pos, int pos0,
                        double base, double freq_scale, const float *freqs, hipStream_t st);

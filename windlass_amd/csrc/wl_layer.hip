@@ -12,6 +12,8 @@
 #include "wl_attention.h"
 #include "wl_layer.h"
 
+#include "wl_frag.h"
+
 #include "wl_device.h"
 
 #include <math.h>
@@ -61,13 +63,11 @@ __device__ __forceinline__ double block_sum_dpp(double v, double *sh) {
 // its values in double (float4 loads when the row allows), then a tree over the workgroup.
 // Enough threads that a thread holds a few loads at most: the row's latency is one or two
 // memory round trips, not a chain of them.
-__global__ __launch_bounds__(1024) void rms_norm_kernel(const float *x, int64_t dim, const float *__restrict__ w,
-                                                        float eps, float *y) {  // x == y allowed
+// put4(i, v): the four results from value i (vec rows), put1(i, v): one.
+template <class Put>
+__device__ __forceinline__ void rms_row(const float *xr, int64_t dim, const float *__restrict__ w, float eps, bool vec,
+                                        const Put &put) {
   __shared__ double sh[16];
-  const float *xr = x + (int64_t)blockIdx.x * dim;
-  float *yr = y + (int64_t)blockIdx.x * dim;
-  const bool vec = (dim & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
-                   ((uintptr_t)w & 15) == 0;
   double s = 0.0;
   if (vec && dim <= (int64_t)blockDim.x * 8) {
     // at most two float4 per thread: x and w both loaded before the reduction, one round trip
@@ -93,11 +93,9 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(const float *x, int64_t 
     const float mean = (float)(s / (double)dim);
     const float scale = 1.0f / (float)sqrt((double)(mean + eps));
     if (i0 < dim)
-      *reinterpret_cast<float4 *>(yr + i0) =
-          make_float4(xa.x * scale * wa.x, xa.y * scale * wa.y, xa.z * scale * wa.z, xa.w * scale * wa.w);
+      put.put4(i0, make_float4(xa.x * scale * wa.x, xa.y * scale * wa.y, xa.z * scale * wa.z, xa.w * scale * wa.w));
     if (i1 < dim)
-      *reinterpret_cast<float4 *>(yr + i1) =
-          make_float4(xb.x * scale * wb.x, xb.y * scale * wb.y, xb.z * scale * wb.z, xb.w * scale * wb.w);
+      put.put4(i1, make_float4(xb.x * scale * wb.x, xb.y * scale * wb.y, xb.z * scale * wb.z, xb.w * scale * wb.w));
     return;
   }
   if (vec) {
@@ -117,12 +115,44 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(const float *x, int64_t 
   if (vec) {
     for (int64_t i = (int64_t)threadIdx.x * 4; i < dim; i += (int64_t)blockDim.x * 4) {
       const float4 v = *reinterpret_cast<const float4 *>(xr + i), g = *reinterpret_cast<const float4 *>(w + i);
-      *reinterpret_cast<float4 *>(yr + i) =
-          make_float4(v.x * scale * g.x, v.y * scale * g.y, v.z * scale * g.z, v.w * scale * g.w);
+      put.put4(i, make_float4(v.x * scale * g.x, v.y * scale * g.y, v.z * scale * g.z, v.w * scale * g.w));
     }
   } else {
-    for (int64_t i = threadIdx.x; i < dim; i += blockDim.x) yr[i] = xr[i] * scale * w[i];
+    for (int64_t i = threadIdx.x; i < dim; i += blockDim.x) put.put1(i, xr[i] * scale * w[i]);
   }
+}
+
+struct PutRow {
+  float *y;
+  __device__ void put4(int64_t i, float4 v) const { *reinterpret_cast<float4 *>(y + i) = v; }
+  __device__ void put1(int64_t i, float v) const { y[i] = v; }
+};
+
+__global__ __launch_bounds__(1024) void rms_norm_kernel(const float *x, int64_t dim, const float *__restrict__ w,
+                                                        float eps, float *y) {  // x == y allowed
+  const bool vec = (dim & 3) == 0 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)y & 15) == 0 &&
+                   ((uintptr_t)w & 15) == 0;
+  rms_row(x + (int64_t)blockIdx.x * dim, dim, w, eps, vec, PutRow{y + (int64_t)blockIdx.x * dim});
+}
+
+// The row's results as the bf16 pieces of the products that read them (wl_frag.h): what a prompt's
+// norm wrote in fp32 was read once more to be rounded (a launch of 5 us at 45 tokens, 9 at 2,048).
+// Pieces of tokens past the last row stay unwritten: products of those tokens are never stored.
+struct PutFrag {
+  uint16_t *xf;
+  int t, dim, ord;
+  __device__ void put4(int64_t i, float4 v) const {
+    typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+    const b4 o = {(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};  // round to nearest even
+    *reinterpret_cast<b4 *>(xf + frag_at(t, (int)i & ~7, dim, ord) * 8 + (i & 4)) = o;
+  }
+  __device__ void put1(int64_t, float) const {}  // rows of whole 256-value blocks only
+};
+
+__global__ __launch_bounds__(1024) void rms_norm_frag_kernel(const float *__restrict__ x, int dim,
+                                                             const float *__restrict__ w, float eps, int ord,
+                                                             uint16_t *__restrict__ xf) {
+  rms_row(x + (int64_t)blockIdx.x * dim, dim, w, eps, true, PutFrag{xf, (int)blockIdx.x, dim, ord});
 }
 
 // The angle of rotated pair i at a position: RopeTable's running product in double
@@ -889,6 +919,20 @@ hipError_t rms_norm_launch(const float *x, int64_t rows, int64_t dim, const floa
   int nt = (int)((dim / 4 + 63) / 64 * 64);  // a float4 per thread, 64..1024 threads
   nt = nt < 64 ? 64 : nt > 1024 ? 1024 : nt;
   hipLaunchKernelGGL(rms_norm_kernel, dim3((unsigned)rows), dim3(nt), 0, st, x, dim, w, eps, y);
+  return hipGetLastError();
+}
+
+bool rms_norm_frag_applies(const float *x, int64_t dim, const float *w) {
+  return dim % 256 == 0 && dim <= 1 << 24 && ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0;
+}
+
+hipError_t rms_norm_frag_launch(const float *x, int rows, int64_t dim, const float *w, float eps, int ord, void *xf,
+                                hipStream_t st) {
+  if (rows <= 0) return hipSuccess;
+  if (!rms_norm_frag_applies(x, dim, w)) return hipErrorInvalidValue;
+  const int nt = dim >= 4096 ? 1024 : (int)(dim / 4);  // as rms_norm_launch: the same sums
+  hipLaunchKernelGGL(rms_norm_frag_kernel, dim3((unsigned)rows), dim3(nt), 0, st, x, (int)dim, w, eps, ord,
+                     (uint16_t *)xf);
   return hipGetLastError();
 }
 
