@@ -1,4 +1,4 @@
-"""Prompts of 9 to 128 tokens (Transformer.MatMul past 8 tokens, src/Transformer.cs:526-536) on the
+"""Prompts of 9 tokens and more over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows. 9 to 128 tokens (Transformer.MatMul past 8 tokens, src/Transformer.cs:526-536) on the
 kernel that reads and decodes each weight once for all tokens: at the edges of its 16-token tiles
 and 16- and 32-row groups, with fewer column blocks than waves, and inside a layer, where the
 matrices that share x run in one launch and the norm and the SiLU write the operands."""
@@ -41,6 +41,15 @@ def test_bars(ctx, t, rows, cols, T):
     w.free()
 
 
+# past 128 tokens: one more, the edges of 256- and 512-token tiles, K unsplit and split (one tile of
+# 300 rows over 9 and 17 column blocks, 2,100 rows), a partly filled second tile
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: t.name)
+@pytest.mark.parametrize("rows,cols,T", [(300, 2304, 129), (130, 256, 256), (300, 4352, 257), (2100, 512, 300),
+                                         (129, 1024, 512), (257, 768, 530)])
+def test_long_bars(ctx, t, rows, cols, T):
+    test_bars(ctx, t, rows, cols, T)
+
+
 def P(t):
     return ctypes.c_void_p(t.data_ptr())
 
@@ -48,9 +57,11 @@ def P(t):
 # one order of x for q, k and v (one launch), two (one by one); down of either order
 @pytest.mark.parametrize("qkv,gu,down", [(("Q4_K", "Q5_K", "Q6_K"), "Q4_K", "Q6_K"), (("Q8_0",) * 3, "IQ4_XS", "Q8_0"),
                                          (("Q4_K", "Q8_0", "Q6_K"), "Q6_K", "IQ4_XS")])
-@pytest.mark.parametrize("T", [9, 47, 128])
+@pytest.mark.parametrize("T", [9, 47, 128, 200])
 def test_layer_equals_its_operations(ctx, qkv, gu, down, T):
-    """A prompt's layer gives the bits of its operations called one at a time."""
+    """A prompt's layer gives the bits of its operations called one at a time (past 128 tokens q, k and v
+    may split K otherwise together than alone: the last bit of a sum moves, and some bf16 and fp16
+    roundings with it)."""
     L, h, rng = load(), ctx.handle, np.random.default_rng(T)
     E, H, KH, HD, FF, pos0 = 512, 4, 2, 64, 768, 3
     mats = {"attn_q": (qkv[0], H * HD, E), "attn_k": (qkv[1], KH * HD, E), "attn_v": (qkv[2], KH * HD, E),
@@ -91,9 +102,14 @@ def test_layer_equals_its_operations(ctx, qkv, gu, down, T):
     mm("ffn_down", h32, o)
     check(L.wl_residual_dev(h, P(xb), P(o), T * E, f(0.5)))
     ctx.sync()
-    assert torch.equal(Ka, Kb) and torch.equal(Va, Vb)
+    if T <= 128:
+        assert torch.equal(Ka, Kb) and torch.equal(Va, Vb)
+    else:  # fp16 values one step apart at most
+        for a, b in ((Ka, Kb), (Va, Vb)):
+            a, b = a.view(torch.float16).float(), b.view(torch.float16).float()
+            assert bool(((a - b).abs() <= 2.0 ** -10 * b.abs() + 2.0 ** -14).all())
     # h is rounded to bf16: a last-bit difference between the two exponentials moves few values by one step
     diff = (xa - xb).abs()
-    assert float((diff > 0).float().mean()) < 0.02 and float(diff.max()) <= 2.0 ** -8 * float(xb.abs().max())
+    assert (T > 128 or float((diff > 0).float().mean()) < 0.02) and float(diff.max()) <= 2.0 ** -8 * float(xb.abs().max())
     for m in w.values():
         m.free()

@@ -638,25 +638,68 @@ static int intdot_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int
   return int_run(c, w, base, nullptr, rows, d_x, acts, T, d_y, fixed);
 }
 
-// A prompt of 9 to 128 tokens (wl_gemm_short.h): x as pieces, then the products, added into d_y
-// times rs with add.
-static size_t short_bytes(const wl_weight *w, int T) {
-  return (size_t)wl::frag_bytes(T, (int)w->cols, wl::short_order(w->type));
+// Prompts over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows: 9 to 128 tokens (wl_gemm_short.h), more
+// (wl_gemm_tall.hip). x goes to bf16 pieces in the order the kernel reads, then the products.
+static bool prompt_applies(const wl_weight *w, int T) {
+  return wl::short_applies(w->type, T, w->cols) || (wl::gemm_tall_applies(w->type, T) && w->cols % 256 == 0);
 }
 
-static wl::ShortMat short_mat(const wl_weight *w, float *d_y) {
-  return wl::ShortMat{w->dev, w->row_bytes, (int)w->rows, w->type, d_y, w->rows};
+static int prompt_order(const wl_weight *w, int T) { return T > 128 ? 2 : wl::short_order(w->type); }
+
+static size_t prompt_bytes(const wl_weight *w, int T) {
+  return (size_t)wl::frag_bytes(T, (int)w->cols, prompt_order(w, T));
 }
 
-static int short_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int64_t rows, const float *d_x, int T,
-                        float *d_y, bool add, float rs, void *fixed) {
-  const int cols = (int)w->cols;
-  void *xf = nullptr;
-  if (int rc = scratch_for(c, S_XB, short_bytes(w, T), fixed, &xf)) return rc;
-  WL_HIP(wl::short_frag_launch(d_x, T, cols, wl::short_order(w->type), xf, c->stream), "gemm operands");
-  const wl::ShortMat m{base, w->row_bytes, (int)rows, w->type, d_y, rows};
-  WL_HIP(wl::short_matmul_launch(&m, 1, cols, xf, T, add, rs, c->num_cu, c->stream), "gemm launch");
+static hipError_t prompt_pieces(const float *d_x, int T, int cols, int ord, void *xf, hipStream_t st) {
+  return ord == 2 ? wl::tall_frag_launch(d_x, T, cols, xf, st) : wl::short_frag_launch(d_x, T, cols, ord, xf, st);
+}
+
+// A product of a launch: y = W x of rows of W from base on.
+struct PromptMat {
+  const wl_weight *w;
+  const uint8_t *base;
+  int rows;
+  float *y;
+};
+
+static void tall_mats(const PromptMat *m, int n, wl::TallMat *s) {
+  for (int i = 0; i < n; i++) s[i] = wl::TallMat{m[i].base, m[i].w->row_bytes, m[i].rows, m[i].w->type, m[i].y, m[i].rows};
+}
+
+// Up to three products of one x (its pieces at xf, in S_XB or the static scratch), added into their
+// y times rs with add. A long prompt's chunk partials follow the pieces.
+static int64_t prompt_part_bytes(const wl_ctx *c, const PromptMat *m, int n, int T, const void *fixed) {
+  if (T <= 128) return 0;
+  wl::TallMat s[3];
+  tall_mats(m, n, s);
+  const int64_t limit = fixed ? (int64_t)(kStaticScratchBytes - prompt_bytes(m[0].w, T)) : INT64_MAX;
+  return wl::tall_part_bytes(s, n, (int)m[0].w->cols, T, c->num_cu, limit);
+}
+
+static int prompt_products(wl_ctx *c, const PromptMat *m, int n, const void *xf, int T, bool add, float rs, void *part,
+                           int64_t part_bytes) {
+  const int cols = (int)m[0].w->cols;
+  if (T <= 128) {
+    wl::ShortMat s[3];
+    for (int i = 0; i < n; i++) s[i] = wl::ShortMat{m[i].base, m[i].w->row_bytes, m[i].rows, m[i].w->type, m[i].y, m[i].rows};
+    WL_HIP(wl::short_matmul_launch(s, n, cols, xf, T, add, rs, c->num_cu, c->stream), "gemm launch");
+    return WL_OK;
+  }
+  wl::TallMat s[3];
+  tall_mats(m, n, s);
+  WL_HIP(wl::tall_matmul_launch(s, n, cols, xf, T, add, rs, part, part_bytes, c->num_cu, c->stream), "gemm launch");
   return WL_OK;
+}
+
+static int prompt_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int64_t rows, const float *d_x, int T,
+                         float *d_y, bool add, float rs, void *fixed) {
+  const PromptMat m{w, base, (int)rows, d_y};
+  const size_t xb = prompt_bytes(w, T);
+  const int64_t pb = prompt_part_bytes(c, &m, 1, T, fixed);
+  void *xf = nullptr;
+  if (int rc = scratch_for(c, S_XB, xb + (size_t)pb, fixed, &xf)) return rc;
+  WL_HIP(prompt_pieces(d_x, T, (int)w->cols, prompt_order(w, T), xf, c->stream), "gemm operands");
+  return prompt_products(c, &m, 1, xf, T, add, rs, (uint8_t *)xf + xb, pb);
 }
 
 // fixed: the static scratch (the allocation-free entry point), or null for the context's slots.
@@ -672,8 +715,8 @@ static int matmul_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float
   int64_t rows;
   operand(w, expert, &base, &rows);
   if (int_path(c, w)) return intdot_matmul(c, w, base, rows, d_x, T, d_y, fixed);
-  if (wl::short_applies(w->type, T, w->cols) && (!fixed || short_bytes(w, T) <= kStaticScratchBytes))
-    return short_matmul(c, w, base, rows, d_x, T, d_y, false, 0.f, fixed);
+  if (prompt_applies(w, T) && (!fixed || prompt_bytes(w, T) <= kStaticScratchBytes))
+    return prompt_matmul(c, w, base, rows, d_x, T, d_y, false, 0.f, fixed);
   if (T > 8 && wl::gemm_supports(w->type)) {
     void *xb = nullptr;
     if ((rc = scratch_for(c, S_XB, (size_t)wl::gemm_scratch_bytes(w->type, (int)rows, (int)w->cols, T, c->num_cu), fixed,
@@ -711,7 +754,7 @@ extern "C" int wl_matmul_dev_noalloc(wl_ctx *c, const wl_weight *w, int32_t expe
   return matmul_dev(c, w, expert, d_x, T, d_y, fixed);
 }
 
-// d_y += (W x) * rs. Up to 128 tokens on the float kernels the add is their final store; otherwise
+// d_y += (W x) * rs. On the float kernels that take 8 tokens or prompts the add is their final store; otherwise
 // the product goes to scratch and the residual kernel adds it. Either way o = W x is rounded to
 // float first, then x + o * rs as two roundings (src/Transformer.cs:224,231).
 extern "C" int wl_matmul_add_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float *d_x, int32_t T,
@@ -729,8 +772,7 @@ extern "C" int wl_matmul_add_dev(wl_ctx *c, const wl_weight *w, int32_t expert, 
     m.rs = rs;
     return gemv(c, &m, 1, 1, d_x, (int)w->cols, T);
   }
-  if (wl::short_applies(w->type, T, w->cols) && !int_path(c, w))
-    return short_matmul(c, w, base, rows, d_x, T, d_y, true, rs, nullptr);
+  if (prompt_applies(w, T) && !int_path(c, w)) return prompt_matmul(c, w, base, rows, d_x, T, d_y, true, rs, nullptr);
   if ((rc = ensure(c, S_LO, (size_t)T * rows * sizeof(float)))) return rc;
   float *o = (float *)c->buf[S_LO];
   if ((rc = matmul_dev(c, w, expert, d_x, T, o))) return rc;
@@ -1359,26 +1401,30 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
     }
     return WL_OK;
   };
-  // Prompts of 9 to 128 tokens whose matrices read x in one order: the norm writes x as pieces, the
-  // matrices that share x are one launch, and gate and up write the down product's pieces.
+  // Prompts whose matrices read x in one order: the norm writes x as pieces, the matrices that share x
+  // are one launch, and gate and up (or the SiLU after them) write the down product's pieces.
   auto one_order = [&](const wl_weight *const *ws, int n) {
     for (int i = 0; i < n; i++)
-      if (each || !wl::short_applies(ws[i]->type, T, ws[i]->cols) || int_path(c, ws[i]) || ws[i]->experts != 1 ||
-          wl::short_order(ws[i]->type) != wl::short_order(ws[0]->type))
+      if (each || !prompt_applies(ws[i], T) || int_path(c, ws[i]) || ws[i]->experts != 1 ||
+          prompt_order(ws[i], T) != prompt_order(ws[0], T))
         return false;
     return true;
   };
-  auto pieces = [&](const float *norm, int ord, void **xf) -> int {
-    if (int r = ensure(c, S_XB, (size_t)wl::frag_bytes(T, E, ord))) return r;
-    *xf = c->buf[S_XB];
+  // the products of T rows of d_x (RMS-normed with norm, where given)
+  auto on_x = [&](const float *norm, const PromptMat *m, int n) -> int {
+    const int ord = prompt_order(m[0].w, T);
+    const size_t xb = prompt_bytes(m[0].w, T);
+    const int64_t pb = prompt_part_bytes(c, m, n, T, nullptr);
+    if (int r = ensure(c, S_XB, xb + (size_t)pb)) return r;
+    uint8_t *xf = (uint8_t *)c->buf[S_XB];
     if (norm && wl::rms_norm_frag_applies(d_x, E, norm)) {
-      WL_HIP(wl::rms_norm_frag_launch(d_x, T, E, norm, L->eps, ord, *xf, c->stream), "rms norm");
-      return WL_OK;
+      WL_HIP(wl::rms_norm_frag_launch(d_x, T, E, norm, L->eps, ord, xf, c->stream), "rms norm");
+    } else {
+      if (norm)
+        if (int r = wl_rms_norm_dev(c, d_x, T, E, norm, L->eps, xn)) return r;
+      WL_HIP(prompt_pieces(norm ? xn : d_x, T, E, ord, xf, c->stream), "gemm operands");
     }
-    if (norm)
-      if (int r = wl_rms_norm_dev(c, d_x, T, E, norm, L->eps, xn)) return r;
-    WL_HIP(wl::short_frag_launch(norm ? xn : d_x, T, E, ord, *xf, c->stream), "gemm operands");
-    return WL_OK;
+    return m[0].y ? prompt_products(c, m, n, xf, T, false, 0.f, xf + xb, pb) : WL_OK;
   };
   // attention block (x itself is the input under post-norms: OLMo 2 has no pre-norm)
   const float *ain = post ? d_x : xn;
@@ -1386,10 +1432,8 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
   const bool qkv_one = one_order(qkv, 3);
   if (!post && !qkv_one && (rc = wl_rms_norm_dev(c, d_x, T, E, L->d_attn_norm, L->eps, xn))) return rc;
   if (qkv_one) {
-    void *xf;
-    if ((rc = pieces(post ? nullptr : L->d_attn_norm, wl::short_order(L->attn_q->type), &xf))) return rc;
-    const wl::ShortMat m[3] = {short_mat(L->attn_q, q), short_mat(L->attn_k, k), short_mat(L->attn_v, v)};
-    WL_HIP(wl::short_matmul_launch(m, 3, E, xf, T, false, 0.f, c->num_cu, c->stream), "q, k, v");
+    const PromptMat m[3] = {{qkv[0], qkv[0]->dev, QD, q}, {qkv[1], qkv[1]->dev, KD, k}, {qkv[2], qkv[2]->dev, KD, v}};
+    if ((rc = on_x(post ? nullptr : L->d_attn_norm, m, 3))) return rc;
   } else if (T <= 8 || each) {
     for (int t0 = 0; t0 < T; t0 += 8) {  // q, k, v in one launch per 8 rows
       const int n = T - t0 < 8 ? T - t0 : 8;
@@ -1435,15 +1479,25 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
   const float *fin = post ? d_x : xn;
   const wl_weight *gu[2] = {L->ffn_gate, L->ffn_up};
   if (!moe && !post && L->ffn_gate->type == L->ffn_up->type && one_order(gu, 2) && one_order(&L->ffn_down, 1)) {
-    void *xf;
-    if ((rc = pieces(L->d_ffn_norm, wl::short_order(L->ffn_gate->type), &xf))) return rc;
-    // the pieces of h (2 bytes a value, tokens rounded up to 16) fit T > 8 rows of floats
-    WL_HIP(wl::short_swiglu_launch(short_mat(L->ffn_gate, nullptr), short_mat(L->ffn_up, nullptr), E, xf, T, g,
-                                   wl::short_order(L->ffn_down->type), c->stream),
-           "gate and up");
-    const wl::ShortMat m = short_mat(L->ffn_down, d_x);
-    WL_HIP(wl::short_matmul_launch(&m, 1, (int)FF, g, T, true, rs, c->num_cu, c->stream), "down");
-    return WL_OK;
+    const PromptMat dm{L->ffn_down, L->ffn_down->dev, E, d_x};
+    if (T <= 128) {
+      const PromptMat none{L->ffn_gate, nullptr, 0, nullptr};
+      if ((rc = on_x(L->d_ffn_norm, &none, 1))) return rc;
+      auto sm = [](const wl_weight *w) { return wl::ShortMat{w->dev, w->row_bytes, (int)w->rows, w->type, nullptr, 0}; };
+      // the pieces of h (2 bytes a value, tokens rounded up to 16) fit T > 8 rows of floats
+      WL_HIP(wl::short_swiglu_launch(sm(L->ffn_gate), sm(L->ffn_up), E, c->buf[S_XB], T, g,
+                                     prompt_order(L->ffn_down, T), c->stream),
+             "gate and up");
+      return prompt_products(c, &dm, 1, g, T, true, rs, nullptr, 0);
+    }
+    const PromptMat m[2] = {{L->ffn_gate, L->ffn_gate->dev, (int)FF, g}, {L->ffn_up, L->ffn_up->dev, (int)FF, u}};
+    if ((rc = on_x(L->d_ffn_norm, m, 2))) return rc;
+    const size_t hb = prompt_bytes(L->ffn_down, T);
+    const int64_t pb = prompt_part_bytes(c, &dm, 1, T, nullptr);
+    if ((rc = ensure(c, S_XB, hb + (size_t)pb))) return rc;
+    uint8_t *hf = (uint8_t *)c->buf[S_XB];
+    WL_HIP(wl::tall_silu_frag_launch(g, u, T, (int)FF, hf, c->stream), "silu");
+    return prompt_products(c, &dm, 1, hf, T, true, rs, hf + hb, pb);
   }
   if (!post && (rc = wl_rms_norm_dev(c, d_x, T, E, L->d_ffn_norm, L->eps, xn))) return rc;
   // SwiGlu (src/Transformer.cs:241-251) into y (added into y with add): up to 8 rows (or every

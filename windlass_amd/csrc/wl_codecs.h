@@ -434,6 +434,16 @@ struct IQ4XSc {
 using IQ4XS = IQ4XSc<true>;    // one-token launches, the MoE experts
 using IQ4XSR = IQ4XSc<false>;  // the batched launches
 
+// Four 4-bit indices (one per byte) -> their kvalues_iq4nl as signed bytes.
+__device__ __forceinline__ uint32_t iq4_signed4(uint32_t idx) {
+  constexpr uint32_t F = 0x80808080u;
+  const uint32_t i3 = idx & 0x07070707u;
+  const uint32_t lo = __builtin_amdgcn_perm(IQ4XS::kT1 ^ F, IQ4XS::kT0 ^ F, i3);
+  const uint32_t hi = __builtin_amdgcn_perm(IQ4XS::kT3 ^ F, IQ4XS::kT2 ^ F, i3);
+  const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((idx >> 3) & 0x01010101u) | 0x0C0C0C0Cu);
+  return (hi & m) | (lo & ~m);
+}
+
 // ------------------------------------------------------------------------- IQ2_XXS
 // Lane slice: sub-block ib32 = sub: four groups of 8 values, each a grid entry (8 bytes of
 // 8/25/43) with eight signs from a 7-bit index plus a parity bit.

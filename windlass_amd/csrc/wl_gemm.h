@@ -19,11 +19,22 @@ int64_t gemm_scratch_bytes(int type, int rows, int cols, int T, int num_cu);
 hipError_t gemm_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, int cols, const float *x, int T,
                        float *y, int ldy, void *scratch, int num_cu, hipStream_t st);
 
-// The 512-token tiles for Q4_K / Q6_K prompts of 384 tokens and more (wl_gemm_tall.hip):
-// gemm_launch and gemm_scratch_bytes hand such calls to these.
+// Prompts of more than 128 tokens over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows (wl_gemm_tall.hip): x (or
+// silu(g) * u) as bf16 pieces in order 2 of wl_frag.h, then up to three matrices on them in one
+// launch (y, or y += result * rs), with tall_part_bytes of scratch, at most limit.
 bool gemm_tall_applies(int type, int T);
-int64_t gemm_tall_scratch_bytes(int rows, int cols, int T, int num_cu);
-hipError_t gemm_tall_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, int cols, const float *x, int T,
-                            float *y, int ldy, void *scratch, int num_cu, hipStream_t st);
+constexpr int TALL_MAX_MATS = 3;
+struct TallMat {
+  const uint8_t *w;
+  int64_t row_bytes;
+  int rows, type;
+  float *y;
+  int64_t ldy;
+};
+hipError_t tall_frag_launch(const float *x, int T, int cols, void *xf, hipStream_t st);
+hipError_t tall_silu_frag_launch(const float *g, const float *u, int T, int cols, void *xf, hipStream_t st);
+int64_t tall_part_bytes(const TallMat *mats, int n, int cols, int T, int num_cu, int64_t limit);
+hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *xf, int T, bool add, float rs,
+                              void *part, int64_t limit, int num_cu, hipStream_t st);
 
 }  // namespace wl

@@ -381,7 +381,6 @@ int gemm_chunks(int type, int rows, int cols, int T, int num_cu) {
 }
 
 int64_t gemm_scratch_bytes(int type, int rows, int cols, int T, int num_cu) {
-  if (gemm_tall_applies(type, T)) return gemm_tall_scratch_bytes(rows, cols, T, num_cu);
   const int S = gemm_chunks(type, rows, cols, T, num_cu);
   return (int64_t)T * cols * 2 + (S > 1 ? (int64_t)S * T * rows * 4 : 0);
 }
@@ -418,8 +417,6 @@ hipError_t gemm_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, 
                        float *y, int ldy, void *scratch, int num_cu, hipStream_t st) {
   if (rows <= 0 || T <= 0) return hipSuccess;
   if (cols <= 0 || cols % 256 || !scratch) return hipErrorInvalidValue;
-  if (gemm_tall_applies(type, T))
-    return gemm_tall_launch(type, w, row_bytes, rows, cols, x, T, y, ldy, scratch, num_cu, st);
   const int64_t n4 = (int64_t)T * cols / 4;
   int64_t g = (n4 + 255) / 256;
   if (g > 4096) g = 4096;

@@ -124,20 +124,6 @@ struct SQ5K {
   }
 };
 
-// Blocks sit at 2-byte alignment: their fields come with loads of that alignment, which the
-// hardware takes at any address.
-typedef uint32_t u32x4a2_t __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2a2_t __attribute__((ext_vector_type(2), aligned(2)));
-__device__ __forceinline__ uint4 ld16_a2(const uint8_t *p) {
-  const u32x4a2_t v = *reinterpret_cast<const u32x4a2_t *>(p);
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint2 ld8_a2(const uint8_t *p) {
-  const u32x2a2_t v = *reinterpret_cast<const u32x2a2_t *>(p);
-  return make_uint2(v.x, v.y);
-}
-__device__ __forceinline__ uint32_t ld2(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
-
 // s * v of the eight signed bytes of a, b (a product rounds once: the order of its factors is free)
 __device__ __forceinline__ uint4 scaled_chunk(float s, uint32_t a, uint32_t b) {
   a = whole(a);
@@ -152,11 +138,11 @@ struct SQ6K {
   struct Scale { float ds[4]; };
   __device__ static void load(const uint8_t *b, int q, Raw &r) {
     const int hh = q >> 1, ih = q & 1;
-    r.l0 = ld16_a2(b + 64 * hh + 16 * ih);
-    r.l1 = ld16_a2(b + 64 * hh + 32 + 16 * ih);
-    r.qh = ld16_a2(b + 128 + 32 * hh + 16 * ih);
-    r.sc = ld8_a2(b + 192 + 8 * hh);
-    r.d = ld2(b + 208);
+    r.l0 = ldw16_a2(b + 64 * hh + 16 * ih);
+    r.l1 = ldw16_a2(b + 64 * hh + 32 + 16 * ih);
+    r.qh = ldw16_a2(b + 128 + 32 * hh + 16 * ih);
+    r.sc = ldw8_a2(b + 192 + 8 * hh);
+    r.d = ldw2(b + 208);
   }
   __device__ static Scale scale(const Raw &r, int q) {
     const float d = half_lo(r.d);
@@ -186,9 +172,9 @@ struct SQ80 {
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       const uint8_t *b = blk + 68 * q + 34 * i;
-      r.d[i] = ld2(b);
-      r.v[2 * i] = ld16_a2(b + 2);
-      r.v[2 * i + 1] = ld16_a2(b + 18);
+      r.d[i] = ldw2(b);
+      r.v[2 * i] = ldw16_a2(b + 2);
+      r.v[2 * i + 1] = ldw16_a2(b + 18);
     }
   }
   __device__ static Scale scale(const Raw &r, int) { return Scale{{half_lo(r.d[0]), half_lo(r.d[1])}}; }
@@ -203,20 +189,11 @@ struct SIQ4XS {
   static constexpr int BYTES = 136;
   struct Raw { uint2 h, v[4]; };
   struct Scale { float dl[2]; };
-  // kvalues_iq4nl as signed bytes
-  __device__ static uint32_t lookup(uint32_t idx) {
-    constexpr uint32_t F = 0x80808080u;
-    const uint32_t i3 = idx & 0x07070707u;
-    const uint32_t lo = __builtin_amdgcn_perm(IQ4XS::kT1 ^ F, IQ4XS::kT0 ^ F, i3);
-    const uint32_t hi = __builtin_amdgcn_perm(IQ4XS::kT3 ^ F, IQ4XS::kT2 ^ F, i3);
-    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((idx >> 3) & 0x01010101u) | 0x0C0C0C0Cu);
-    return (hi & m) | (lo & ~m);
-  }
   __device__ static void load(const uint8_t *b, int q, Raw &r) {  // 8-byte aligned
     r.h = ldw8(b);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
-      const uint4 v = ld16_a2(b + 8 + 32 * q + 16 * i);
+      const uint4 v = ldw16_a2(b + 8 + 32 * q + 16 * i);
       r.v[2 * i] = make_uint2(v.x, v.y);
       r.v[2 * i + 1] = make_uint2(v.z, v.w);
     }
@@ -232,7 +209,7 @@ struct SIQ4XS {
   __device__ static uint4 frag(const Raw &r, const Scale &s, int, int m) {
     const int g = m >> 1, p = m & 1;
     const uint2 w = r.v[2 * (g >> 1) + p];
-    return scaled_chunk(s.dl[g >> 1], lookup((w.x >> (4 * (g & 1))) & 0x0F0F0F0Fu), lookup((w.y >> (4 * (g & 1))) & 0x0F0F0F0Fu));
+    return scaled_chunk(s.dl[g >> 1], iq4_signed4((w.x >> (4 * (g & 1))) & 0x0F0F0F0Fu), iq4_signed4((w.y >> (4 * (g & 1))) & 0x0F0F0F0Fu));
   }
 };
 

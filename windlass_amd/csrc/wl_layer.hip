@@ -200,41 +200,53 @@ __global__ __launch_bounds__(64) void rope_table_kernel(float4 *__restrict__ tab
 
 // RoPE on q (H heads) and k (KH heads) of row t, and ToHalf of the row's keys and values into
 // cache row pos0 + t, or row pos[t] of slot slot[t] (slots of cap positions) for a batch step
-// (src/Transformer.cs:204-215,342-348). Work items of a row: one per rotated pair of every q and
-// k head, then one per key/value column (the value's store, and the key's for columns past
-// rope_dims). k, v and the caches are null for RoPE on one tensor.
+// (src/Transformer.cs:204-215,342-348). A workgroup takes the angles of 256 pairs of its row once, into
+// LDS (a thread per pair; a thread per pair and head took the double cosine and sine H + KH times:
+// 2,048 rows of 40 heads 90 us), then a thread per rotated pair of the q and k heads and per key/value
+// column (the value's store, and the key's for columns past rope_dims), both shared by the gridDim.y
+// workgroups of a row. k, v and the caches are null for RoPE on one tensor.
 __global__ __launch_bounds__(256) void rope_qkv_kernel(float *__restrict__ q, int64_t ldq, int H, float *__restrict__ k,
                                                        const float *__restrict__ v, int KH, int hd, int n, int neox,
                                                        const int *__restrict__ pos, int pos0, double theta_scale,
                                                        double freq_scale, const float *__restrict__ freqs,
                                                        uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc,
                                                        const int *__restrict__ slot, int64_t cap) {
-  const int t = blockIdx.y, half = n / 2, KD = KH * hd;
-  const int it = blockIdx.x * blockDim.x + threadIdx.x;
-  const int npairs = (H + KH) * half;
+  __shared__ float2 angle[256];  // (cos, sin)
+  const int t = blockIdx.x, half = n / 2, KD = KH * hd, tid = threadIdx.x;
+  const int first = blockIdx.y * 256 + tid, step = gridDim.y * 256;
   const int p = pos ? pos[t] : pos0 + t;
   const int64_t crow = (slot ? (int64_t)slot[t] * cap + p : (int64_t)(pos0 + t)) * KD;
-  float c = 0.f, s = 0.f;  // every lane runs the angle product (uniform trip count)
-  if (half > 0) rope_cs(p, it < npairs ? it % half : 0, half, theta_scale, freq_scale, freqs, c, s);
-  if (it < npairs) {
-    const int head = it / half, i = it % half;
-    float y0, y1;
-    int a, b;
-    if (head < H) {
-      rope_pair(q + (int64_t)t * ldq + (int64_t)head * hd, i, n, neox, c, s, y0, y1, a, b);
-    } else {
-      const int kh = head - H;
-      rope_pair(k + (int64_t)t * KD + (int64_t)kh * hd, i, n, neox, c, s, y0, y1, a, b);
-      if (Kc) {
-        Kc[crow + kh * hd + a] = to_half(y0);
-        Kc[crow + kh * hd + b] = to_half(y1);
+  for (int i0 = 0; i0 < half; i0 += 256) {
+    const int cn = min(256, half - i0);
+    if (i0) __syncthreads();  // the pairs before are rotated
+    if ((tid & ~63) < cn) {   // whole waves run the angle product (uniform trip count)
+      float c, s;
+      rope_cs(p, tid < cn ? i0 + tid : 0, half, theta_scale, freq_scale, freqs, c, s);
+      if (tid < cn) angle[tid] = make_float2(c, s);
+    }
+    __syncthreads();
+    for (int it = first; it < (H + KH) * cn; it += step) {
+      const int head = it / cn, i = i0 + it % cn;
+      const float2 cs = angle[it % cn];
+      float y0, y1;
+      int a, b;
+      if (head < H) {
+        rope_pair(q + (int64_t)t * ldq + (int64_t)head * hd, i, n, neox, cs.x, cs.y, y0, y1, a, b);
+      } else {
+        const int kh = head - H;
+        rope_pair(k + (int64_t)t * KD + (int64_t)kh * hd, i, n, neox, cs.x, cs.y, y0, y1, a, b);
+        if (Kc) {
+          Kc[crow + kh * hd + a] = to_half(y0);
+          Kc[crow + kh * hd + b] = to_half(y1);
+        }
       }
     }
-  } else if (it < npairs + KD && Vc) {
-    const int j = it - npairs;
-    Vc[crow + j] = to_half(v[(int64_t)t * KD + j]);
-    if (j % hd >= n) Kc[crow + j] = to_half(k[(int64_t)t * KD + j]);
   }
+  if (Vc)
+    for (int j = first; j < KD; j += step) {
+      Vc[crow + j] = to_half(v[(int64_t)t * KD + j]);
+      if (j % hd >= n) Kc[crow + j] = to_half(k[(int64_t)t * KD + j]);
+    }
 }
 
 // ToHalf (src/Transformer.cs:342-348) of one token's keys and values.
@@ -936,11 +948,13 @@ hipError_t rms_norm_frag_launch(const float *x, int rows, int64_t dim, const flo
   return hipGetLastError();
 }
 
+// Workgroups of a row: few rows spread over the CUs, many take their angles once.
+static unsigned rope_split(int T) { return T >= 512 ? 1 : T >= 128 ? 2 : 8; }
+
 hipError_t rope_launch(float *x, int64_t ldx, int T, int heads, int hd, int n, int neox, const int *pos, int pos0,
                        double base, double freq_scale, const float *freqs, hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  const int64_t items = (int64_t)heads * (n / 2);
-  hipLaunchKernelGGL(rope_qkv_kernel, dim3(blocks_of(items, 256), T), dim3(256), 0, st, x, ldx, heads, nullptr,
+  hipLaunchKernelGGL(rope_qkv_kernel, dim3((unsigned)T, rope_split(T)), dim3(256), 0, st, x, ldx, heads, nullptr,
                      nullptr, 0, hd, n, neox, pos, pos0, pow(base, -2.0 / n), freq_scale, freqs, nullptr, nullptr,
                      nullptr, (int64_t)0);
   return hipGetLastError();
@@ -950,8 +964,7 @@ hipError_t rope_kv_launch(float *q, float *k, const float *v, int T, int H, int 
                           int pos0, double base, double freq_scale, const float *freqs, uint16_t *Kc, uint16_t *Vc,
                           const RowMap &rm, hipStream_t st) {
   if (T <= 0) return hipSuccess;
-  const int64_t items = (int64_t)(H + KH) * (n / 2) + (int64_t)KH * hd;
-  hipLaunchKernelGGL(rope_qkv_kernel, dim3(blocks_of(items, 256), T), dim3(256), 0, st, q, (int64_t)H * hd, H, k, v,
+  hipLaunchKernelGGL(rope_qkv_kernel, dim3((unsigned)T, rope_split(T)), dim3(256), 0, st, q, (int64_t)H * hd, H, k, v,
                      KH, hd, n, neox, rm.pos, pos0, pow(base, -2.0 / n), freq_scale, freqs, Kc, Vc, rm.slot, rm.cap);
   return hipGetLastError();
 }
