@@ -278,10 +278,11 @@ static uint64_t IQ2S_GRID[1024];
 static uint32_t IQ3S_GRID[512];
 static uint8_t KSIGNS[128];
 
-static void tables_init(void)
+/* Run once when the library is loaded, before any thread: filled on first use, a thread of the
+ * first parallel product could find IQ2XXS_GRID[0] set and read the other tables half filled. */
+__attribute__((constructor)) static void tables_init(void)
 {
     static const uint8_t vals[3] = { 0x08, 0x19, 0x2b };
-    if (IQ2XXS_GRID[0]) return;
     for (int i = 0; i < 128; i++) {
         /* ksigns_iq2xs[i]: i plus an eighth bit that makes the bit count even (src/IqTables.cs:10-21). */
         KSIGNS[i] = (uint8_t)(i | ((__builtin_popcount(i) & 1) << 7));
@@ -303,10 +304,10 @@ static void tables_init(void)
     }
 }
 
-const uint64_t *wlo_iq2xxs_grid(void) { tables_init(); return IQ2XXS_GRID; }
-const uint64_t *wlo_iq2s_grid(void) { tables_init(); return IQ2S_GRID; }
-const uint32_t *wlo_iq3s_grid(void) { tables_init(); return IQ3S_GRID; }
-const uint8_t *wlo_ksigns_iq2xs(void) { tables_init(); return KSIGNS; }
+const uint64_t *wlo_iq2xxs_grid(void) { return IQ2XXS_GRID; }
+const uint64_t *wlo_iq2s_grid(void) { return IQ2S_GRID; }
+const uint32_t *wlo_iq3s_grid(void) { return IQ3S_GRID; }
+const uint8_t *wlo_ksigns_iq2xs(void) { return KSIGNS; }
 const int8_t *wlo_kvalues_iq4nl(void) { return KVALUES; }
 
 /* ------------------------------------------------------------ decoders (src/Quants.cs) */
@@ -542,7 +543,6 @@ static void dec_iq4_xs(const uint8_t *b, int64_t n, float *y)
 /* src/IQuants.cs:147-170: db = d * (0.5 + scale4) * 0.25, y = db * gridbyte * sign. */
 static void dec_iq2_xxs(const uint8_t *b, int64_t n, float *y)
 {
-    tables_init();
     for (int64_t i = 0; i < n / 256; i++, b += 66) {
         float d = H(b);
         const uint8_t *qs = b + 2;
@@ -565,7 +565,6 @@ static void dec_iq2_xxs(const uint8_t *b, int64_t n, float *y)
  * grid entry gives 4 values, each sign byte 8. */
 static void dec_iq3_s(const uint8_t *b, int64_t n, float *y)
 {
-    tables_init();
     for (int64_t i = 0; i < n / 256; i++, b += 110) {
         float d = H(b);
         const uint8_t *qs = b + 2, *qh = b + 66, *signs = b + 74, *scales = b + 106;
@@ -597,7 +596,6 @@ static void dec_iq3_s(const uint8_t *b, int64_t n, float *y)
  * qs byte plus two qh bits (10 bits); one sign byte per 8 values. */
 static void dec_iq2_s(const uint8_t *b, int64_t n, float *y)
 {
-    tables_init();
     for (int64_t i = 0; i < n / 256; i++, b += 82) {
         float d = H(b);
         const uint8_t *qs = b + 2, *signs = b + 34, *qh = b + 66, *scales = b + 74;
