@@ -83,6 +83,44 @@ struct WQ4K {
   __device__ static float dmin(const Raw &r) { return half_hi(r.h.x); }
 };
 
+// Q4_K centred: (n - 8) sc, exact (at most 8 * 63), and per sub-block the factor 8 d sc - dmin m of its
+// sum of x, rounded once (both products are exact in fp32).
+struct WQ4KC {
+  static constexpr int BYTES = 144, NF = 1;
+  static constexpr bool MINS = true, SWAP = true;
+  typedef WQ4K::Raw Raw;
+  struct Scale { fh2 sl, sh; float mlo, mhi; };
+
+  __device__ static int xoff4(int q, int m, int h) { return WQ4K::xoff4(q, m, h); }
+  __device__ static void load(const uint8_t *blk, int q, Raw &r) { WQ4K::load(blk, q, r); }
+
+  __device__ static Scale scale(const Raw &r, int q) {
+    const uint4 h = r.h;
+    const int k = 16 * (q & 1);
+    const uint32_t S = q < 2 ? (h.y & 0x3F3F3F3Fu) : ((h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u));
+    const uint32_t M = q < 2 ? (h.z & 0x3F3F3F3Fu) : (((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u));
+    const float sclo = (float)((S >> k) & 0xFF), schi = (float)((S >> (k + 8)) & 0xFF);
+    const float mlo = (float)((M >> k) & 0xFF), mhi = (float)((M >> (k + 8)) & 0xFF);
+    const float dv = d(r), dm = half_hi(r.h.x);
+    const _Float16 a = (_Float16)sclo, b = (_Float16)(schi * 0.0625f);
+    return Scale{fh2{a, a}, fh2{b, b}, __builtin_fmaf(8.f * sclo, dv, -(dm * mlo)),
+                 __builtin_fmaf(8.f * schi, dv, -(dm * mhi))};
+  }
+
+  __device__ static void frag(const Raw &r, const Scale &s, int, int m, fh8 (&f)[1]) {
+    const uint32_t qd[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
+    const uint32_t D = qd[m], D8 = D >> 8;
+    // 1024 + n - 1032 and 1024 + 16 n - 1152
+    const fh2 L = {(_Float16)-1032.f, (_Float16)-1032.f}, H = {(_Float16)-1152.f, (_Float16)-1152.f};
+    const fh2 p0 = (as_fh2((D & 0x000F000Fu) | 0x64006400u) + L) * s.sl;
+    const fh2 p1 = (as_fh2((D8 & 0x000F000Fu) | 0x64006400u) + L) * s.sl;
+    const fh2 p2 = (as_fh2((D & 0x00F000F0u) | 0x64006400u) + H) * s.sh;
+    const fh2 p3 = (as_fh2((D8 & 0x00F000F0u) | 0x64006400u) + H) * s.sh;
+    f[0] = fh8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+  }
+  __device__ static float d(const Raw &r) { return half_lo(r.h.x); }
+};
+
 // ------------------------------------------------------------------------------------ Q6_K
 // Quarter q = 2hh + ih of a super-block: half hh (128 values), i in [16 ih, 16 ih + 16) of its
 // four 32-value groups g, whose 6-bit values are ql[64hh + i] (g 0, 2: low, high nibble) or

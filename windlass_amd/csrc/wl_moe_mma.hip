@@ -9,10 +9,13 @@
 //
 // Arithmetic, at fp32's precision: a weight is an exact fp16 integer (wl_fmma_codec.h), a
 // token's 256 activations of a super-block are scaled by a power of two and split into
-// hi = fp16(x f), lo = fp16(x f - hi), 22 significant bits, and both products accumulate exactly
-// into fp32. Q4_K's minimum is a 16x16x4 fp32 MFMA of the rows' mins with the sub-blocks' sums of
-// x. A super-block's sum is then scaled by d and 1/f and added in order, so a token's result
-// depends neither on the other tokens nor on its place in a tile.
+// hi = fp16(x f), lo = fp16(x f - hi), 22 significant bits, and the exact products accumulate into
+// fp32, the parts apart (the lo sums round 2^11 times finer). Q4_K's quants enter as n - 8, with the
+// sub-block's 8 d sc - dmin m as the factor of its sum of x (a 16x16x4 fp32 MFMA): the two large
+// terms that nearly cancel in n sc and the minimum never become sums of their own (error against 64
+// bits at 300 tokens of 128 experts 5.2e-7 with n, 3.7e-7 row by row in fp32). A super-block's sum is
+// then scaled by d and 1/f and added in order, so a token's result depends neither on the other tokens
+// nor on its place in a tile.
 //
 // Launches: route (one wave per token), plan (one workgroup per expert numbers its pairs), the
 // tokens' parts, gate/up with the SiLU, the hidden rows' parts, down, combine.
@@ -111,7 +114,7 @@ __global__ __launch_bounds__(256) void moe_parts_kernel(const float *__restrict_
   fh8 o;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    // the chunk's order of each four values (WQ4K: 0, 2, 1, 3)
+    // the chunk's order of each four values (WQ4KC: 0, 2, 1, 3)
     const int j = C::SWAP && (i & 3) == 1 ? i + 1 : C::SWAP && (i & 3) == 2 ? i - 1 : i;
     const float X = v[j] * f;
     const _Float16 hi = (_Float16)X;
@@ -231,14 +234,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 #pragma unroll
     for (int w0 = 0; w0 < 2; w0 += G) {
       typename C::Scale sc[G];
-      ff4 acc1[G][NT][C::NF];
+      ff4 acc1[G][NT][C::NF], acc2[G][NT][C::NF];  // the sums of the hi and of the lo parts
 #pragma unroll
       for (int w = 0; w < G; w++) {
         sc[w] = C::scale(cur[w0 + w], q);
 #pragma unroll
         for (int t = 0; t < NT; t++)
 #pragma unroll
-          for (int n = 0; n < C::NF; n++) acc1[w][t][n] = ff4{0.f, 0.f, 0.f, 0.f};
+          for (int n = 0; n < C::NF; n++) acc1[w][t][n] = acc2[w][t][n] = ff4{0.f, 0.f, 0.f, 0.f};
       }
 #pragma unroll
       for (int mm = 0; mm < 8; mm++) {
@@ -254,7 +257,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
 #pragma unroll
             for (int n = 0; n < C::NF; n++) {
               acc1[w][t][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, f[w][n], acc1[w][t][n], 0, 0, 0);
-              acc1[w][t][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, f[w][n], acc1[w][t][n], 0, 0, 0);
+              acc2[w][t][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, f[w][n], acc2[w][t][n], 0, 0, 0);
             }
         }
         if ((mm & 1) || G == 1) __builtin_amdgcn_sched_barrier(0);  // one or two chunks' operands live at a time
@@ -270,14 +273,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void m
             ff4 Mn = {0.f, 0.f, 0.f, 0.f};
             Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum[(q * NT + t) * 16 + rr], sc[w].mlo, Mn, 0, 0, 0);
             Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(xsum[((4 + q) * NT + t) * 16 + rr], sc[w].mhi, Mn, 0, 0, 0);
-            const float dm = C::dmin(cur[w0 + w]);
 #pragma unroll
             for (int i = 0; i < 4; i++)
-              o[i] = __builtin_fmaf(__builtin_fmaf(-dm, Mn[i], d * acc1[w][t][0][i]), iv[i], o[i]);
+              o[i] = __builtin_fmaf(__builtin_fmaf(d, acc1[w][t][0][i] + acc2[w][t][0][i], Mn[i]), iv[i], o[i]);
           } else {
 #pragma unroll
             for (int i = 0; i < 4; i++)
-              o[i] = __builtin_fmaf(d * __builtin_fmaf(16.f, acc1[w][t][1][i], acc1[w][t][0][i]), iv[i], o[i]);
+              o[i] = __builtin_fmaf(d * __builtin_fmaf(16.f, acc1[w][t][1][i] + acc2[w][t][1][i],
+                                                       acc1[w][t][0][i] + acc2[w][t][0][i]),
+                                    iv[i], o[i]);
           }
         }
       }
@@ -381,7 +385,7 @@ static hipError_t parts_launch(int type, const float *x, int64_t rows, int cols,
   const int nsb = cols / 256;
   const dim3 grid((unsigned)((rows * nsb + 3) / 4));
   if (type == 12)
-    hipLaunchKernelGGL(moe_parts_kernel<WQ4K>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
+    hipLaunchKernelGGL(moe_parts_kernel<WQ4KC>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
   else
     hipLaunchKernelGGL(moe_parts_kernel<WQ6K>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
   return hipGetLastError();
@@ -432,7 +436,7 @@ hipError_t moe_many_launch(const MoeLaunch &l, void *scratch, hipStream_t st) {
   g.inv = (const float *)(b + s.xinv);
   g.by_pair = 0;
   g.y = (float *)(b + s.h);
-  e = l.gu_type == 12 ? many_gemm<WQ4K, true>(g, nt, max_tiles, st) : many_gemm<WQ6K, true>(g, nt, max_tiles, st);
+  e = l.gu_type == 12 ? many_gemm<WQ4KC, true>(g, nt, max_tiles, st) : many_gemm<WQ6K, true>(g, nt, max_tiles, st);
   if (e != hipSuccess) return e;
   if ((e = parts_launch(l.d_type, g.y, P, l.ff, b + s.hp, b + s.hsum, b + s.hinv, st)) != hipSuccess) return e;
   MoeGemm d = g;
@@ -447,7 +451,7 @@ hipError_t moe_many_launch(const MoeLaunch &l, void *scratch, hipStream_t st) {
   d.inv = (const float *)(b + s.hinv);
   d.by_pair = 1;
   d.y = (float *)(b + s.y);
-  e = l.d_type == 12 ? many_gemm<WQ4K, false>(d, nt, max_tiles, st) : many_gemm<WQ6K, false>(d, nt, max_tiles, st);
+  e = l.d_type == 12 ? many_gemm<WQ4KC, false>(d, nt, max_tiles, st) : many_gemm<WQ6K, false>(d, nt, max_tiles, st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(moe_many_combine_kernel, dim3((unsigned)(((int64_t)l.T * l.embd / 4 + 255) / 256)), dim3(256), 0, st,
                      m, d.y, l.T, l.k, l.embd, l.out);
