@@ -224,3 +224,59 @@ def test_fmma_leaves_other_formats_alone(ctx):
     w = ctx.upload(t, data, rows, cols)
     assert np.array_equal(_bits(Transformer.MatMul(w, x, 3)), _bits(want))
     w.free()
+
+
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: t.name)
+@pytest.mark.parametrize("T", [9, 13, 16, 21])  # one pass of two token sets, and a pass more
+@pytest.mark.parametrize("rows,cols", [(37, 2304), (4128, 512)])  # fewer tiles than CUs, and more than a round's waves
+def test_fmma_wide_pass_rows_equal_single_token_bitwise(ctx, t, T, rows, cols):
+    g, u = (ctx.upload(t, blocks(t, rows, cols, seed=40 + i), rows, cols) for i in range(2))
+    x = _dev(np.random.default_rng(T).standard_normal((T, cols), dtype=np.float32))
+    y, one = torch.empty((T, rows), device="cuda"), torch.empty((T, rows), device="cuda")
+    torch.cuda.synchronize()
+    L = load()
+    check(L.wl_gate_up_dev(ctx.handle, g.handle, u.handle, -1, _p(x), T, _p(y)))
+    for i in range(T):
+        check(L.wl_gate_up_dev(ctx.handle, g.handle, u.handle, -1, _p(x[i:i + 1]), 1, _p(one[i:i + 1])))
+    ctx.sync()
+    assert np.array_equal(_bits(y.cpu().numpy()), _bits(one.cpu().numpy()))
+    g.free()
+    u.free()
+
+
+@pytest.mark.parametrize("types", [("Q4_K", "Q4_K", "Q6_K", "Q4_K", "Q6_K"), ("Q4_K", "Q8_0", "Q6_K", "Q6_K", "Q8_0")])
+@pytest.mark.parametrize("N", [9, 16, 19])
+def test_fmma_batch_step_rows_equal_their_sequences_bitwise(ctx, types, N):
+    """A stacked step past 8 sequences (passes of 16 where every matrix takes the matrix cores, q/k/v
+    together): each row equals its own sequence's step."""
+    from windlass_amd import LayerDesc
+    rng = np.random.default_rng(N)
+    E, H, KH, HD, FF, cap = 512, 4, 2, 64, 768, 12
+    tq, tk, tv, tg, td = types
+    mats = {"attn_q": (tq, H * HD, E), "attn_k": (tk, KH * HD, E), "attn_v": (tv, KH * HD, E), "attn_output": (tq, E, H * HD),
+            "ffn_gate": (tg, FF, E), "ffn_up": (tg, FF, E), "ffn_down": (td, E, FF)}
+    w = {n: ctx.upload(GgmlType[t], blocks(GgmlType[t], r, c, seed=i), r, c) for i, (n, (t, r, c)) in enumerate(mats.items())}
+    norms = [_dev((1 + 0.1 * rng.standard_normal(E)).astype(np.float32)) for _ in range(2)]
+    d = LayerDesc()
+    for n in mats:
+        setattr(d, n, w[n].handle.value)
+    d.d_attn_norm, d.d_ffn_norm = (v.data_ptr() for v in norms)
+    d.embd, d.heads, d.kv_heads, d.head_dim, d.rope_dims = E, H, KH, HD, HD
+    d.rope_base, d.rope_freq_scale, d.eps, d.residual_scale = 10000.0, 1.0, 1e-6, 0.5
+    x0 = rng.standard_normal((N, E), dtype=np.float32)
+    cache = rng.standard_normal((2, N, cap, KH * HD)).astype(np.float16).view(np.int16)
+    pos, slot = [int(p) for p in rng.integers(0, cap, N)], [(i + 3) % N for i in range(N)]
+    out = []
+    for step in (N, 1):
+        x, K, V = _dev(x0), _dev(cache[0]), _dev(cache[1])
+        torch.cuda.synchronize()
+        for i in range(0, N, step):
+            P, S = (ctypes.c_int32 * step)(*pos[i:i + step]), (ctypes.c_int32 * step)(*slot[i:i + step])
+            check(load().wl_layer_batch_dev(ctx.handle, ctypes.byref(d), _p(x[i:i + step]), step, P, S, N, cap, _p(K), _p(V)))
+        ctx.sync()
+        out.append((x, K, V))
+    for a, b in zip(*out):
+        assert torch.equal(a.view(torch.int16) if a.dtype == torch.int16 else a.view(torch.int32),
+                           b.view(torch.int16) if b.dtype == torch.int16 else b.view(torch.int32))
+    for m in w.values():
+        m.free()

@@ -571,6 +571,12 @@ static int gemv(wl_ctx *c, const wl::GemvMat *mats, int nmat, int nm, const floa
   return WL_OK;
 }
 
+// Tokens of a GEMV pass over rows of this matrix: 8, or 16 where the matrix-core GEMV runs them (a
+// token's bits depend on neither).
+static int gemv_pass(const wl_ctx *c, int type, int64_t cols) {
+  return c->float_mma && wl::fmma_supports(type) && cols % 256 == 0 ? wl::FMMA_MAX_T : 8;
+}
+
 // The integer path runs when it is switched on and the weight has an integer kernel whose
 // activation blocks fit the row (src/Transformer.cs:493).
 static bool int_path(const wl_ctx *c, const wl_weight *w) {
@@ -879,9 +885,10 @@ extern "C" int wl_gate_up_dev(wl_ctx *c, const wl_weight *gate, const wl_weight 
     IntActs acts;
     return int_run(c, gate, gb, ub, rows, d_x, acts, T, d_h);
   }
-  for (int t0 = 0; t0 < T; t0 += 8) {
+  const int pass = gemv_pass(c, gate->type, gate->cols);
+  for (int t0 = 0; t0 < T; t0 += pass) {
     const wl::GemvMat m{gb, ub, gate->row_bytes, (int)rows, gate->type, d_h + (int64_t)t0 * rows, (int)rows};
-    const int Tp = T - t0 < 8 ? T - t0 : 8;
+    const int Tp = T - t0 < pass ? T - t0 : pass;
     if ((rc = gemv(c, &m, 1, 2, d_x + (int64_t)t0 * gate->cols, (int)gate->cols, Tp))) return rc;
   }
   return WL_OK;
@@ -1389,13 +1396,28 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
         *v = (float *)c->buf[S_LV], *att = (float *)c->buf[S_LATT],
         *g = (float *)c->buf[S_LG], *u = (float *)c->buf[S_LU];
   const float rs = L->residual_scale != 0.f ? L->residual_scale : 1.f;
-  // y = W x over the T rows: past 8 rows the GEMM, or with each GEMV passes of 8
+  // GEMV passes of 16 rows for these matrices (with each, past 8 rows)
+  auto wide = [&](const wl_weight *const *ws, int n) {
+    for (int i = 0; i < n; i++)
+      if (!each || T <= 8 || int_path(c, ws[i]) || ws[i]->experts != 1 || gemv_pass(c, ws[i]->type, ws[i]->cols) == 8)
+        return false;
+    return true;
+  };
+  // y = W x over the T rows: past 8 rows the GEMM, or with each GEMV passes of 8 or 16
   auto mm = [&](const wl_weight *w, const float *x, float *y, bool add) -> int {
-    const int step = each ? 8 : T;
+    const bool wd = wide(&w, 1);
+    const int step = wd ? wl::FMMA_MAX_T : each ? 8 : T;
     for (int t0 = 0; t0 < T; t0 += step) {
       const int n = T - t0 < step ? T - t0 : step;
       const float *xs = x + (int64_t)t0 * w->cols;
       float *ys = y + (int64_t)t0 * w->rows;
+      if (wd) {
+        wl::GemvMat m{w->dev, nullptr, w->row_bytes, (int)w->rows, w->type, ys, (int)w->rows};
+        m.add = add;
+        m.rs = rs;
+        if (const int r = gemv(c, &m, 1, 1, xs, (int)w->cols, n)) return r;
+        continue;
+      }
       const int r = add ? wl_matmul_add_dev(c, w, -1, xs, n, ys, rs) : matmul_dev(c, w, -1, xs, n, ys);
       if (r) return r;
     }
@@ -1435,9 +1457,18 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
     const PromptMat m[3] = {{qkv[0], qkv[0]->dev, QD, q}, {qkv[1], qkv[1]->dev, KD, k}, {qkv[2], qkv[2]->dev, KD, v}};
     if ((rc = on_x(post ? nullptr : L->d_attn_norm, m, 3))) return rc;
   } else if (T <= 8 || each) {
-    for (int t0 = 0; t0 < T; t0 += 8) {  // q, k, v in one launch per 8 rows
-      const int n = T - t0 < 8 ? T - t0 : 8;
+    const bool wd = wide(qkv, 3);
+    const int step = wd ? wl::FMMA_MAX_T : 8;
+    for (int t0 = 0; t0 < T; t0 += step) {  // q, k, v in one launch per pass
+      const int n = T - t0 < step ? T - t0 : step;
       float *ys[3] = {q + (int64_t)t0 * QD, k + (int64_t)t0 * KD, v + (int64_t)t0 * KD};
+      if (wd) {
+        wl::GemvMat m[3];
+        for (int i = 0; i < 3; i++)
+          m[i] = wl::GemvMat{qkv[i]->dev, nullptr, qkv[i]->row_bytes, (int)qkv[i]->rows, qkv[i]->type, ys[i], (int)qkv[i]->rows};
+        if ((rc = gemv(c, m, 3, 1, ain + (int64_t)t0 * E, E, n))) return rc;
+        continue;
+      }
       if ((rc = wl_matmul_multi_dev(c, 3, qkv, ain + (int64_t)t0 * E, n, ys))) return rc;
     }
   } else if ((rc = mm(L->attn_q, ain, q, false)) || (rc = mm(L->attn_k, ain, k, false)) ||

@@ -1,4 +1,4 @@
-// wl_fmma.hip - the float decode GEMV on the matrix cores: Q4_K and Q6_K rows times 1-8 tokens
+// wl_fmma.hip - the float decode GEMV on the matrix cores: Q4_K and Q6_K rows times 1-16 tokens
 // of fp32 activations on v_mfma_f32_16x16x32_f16 (Transformer.MatMul / MatMulEach,
 // src/Transformer.cs:483-561, float branch), with a token's result independent of how many
 // tokens share the launch.
@@ -15,11 +15,12 @@
 // minimum term, dmin * sum_j m_j * (sum of x over sub-block j), is a 16x16x4 fp32 MFMA of the
 // rows' mins and the sub-block sums of each part. The partial of (row, token, unit) is
 // (hi sum + lo sum) / f, and a second launch adds the units in order (SiLU for the gate/up pair,
-// the residual add), so every token's bits are the same for T = 1..8.
+// the residual add), so every token's bits are the same for T = 1..16.
 //
 // Layout. A workgroup (eight waves) owns one unit of one matrix: its waves first write the
 // tokens' fp16 parts into LDS in the MFMA operand order (64 KB, plus Q4_K's sub-block sums),
-// then each wave takes 16-row tiles on its own: lane (q = l / 16, rr = l % 16) reads row rr's
+// then each wave takes 16-row tiles on its own (9 to 16 tokens: two such
+// sets of parts in 138 KB, sixteen waves, every weight meeting both sets): lane (q = l / 16, rr = l % 16) reads row rr's
 // quarter q of each super-block and feeds the MFMA's B operand; the A operand (16 columns of x
 // parts) comes from LDS, one 16-byte read per MFMA, conflict-free.
 #include "wl_fmma.h"
@@ -34,7 +35,10 @@ constexpr int FM_UNIT = 2048;                        // columns per unit: 8 supe
 constexpr int FM_NS = 16;                            // MFMA columns (two per token)
 constexpr int FM_XBYTES = 8 * 8 * 4 * FM_NS * 16;    // x parts: [sb][m][q][slot] of 8 halves
 constexpr int FM_SBYTES = 8 * 2 * 4 * FM_NS * 4;     // Q4_K sub-block sums: [sb][half][q][slot]
-constexpr int FM_WAVES = 8;
+constexpr int FM_SET = FM_XBYTES + FM_SBYTES;        // LDS of a token set: 8 tokens
+// Token sets of a launch (TS): 1 to 8 tokens, or 9 to 16 whose two sets share each weight's load and
+// unpack (two passes of 8 read and unpacked every weight twice). A wave per token.
+constexpr int fm_waves(int ts) { return 8 * ts; }
 
 // One token's parts of one unit, by one wave: lane (sb = l / 8, e = l % 8) reads 32 values,
 // the wave takes the largest finite |x|, and the lane writes its values' hi and lo halves to
@@ -133,8 +137,9 @@ struct FQ4K {
     r.q1 = ldw16(blk + 32 + 32 * q);
   }
 
-  // acc (columns 4q..4q+3 of row rr) += d * sum(n * sc * x) - dmin * sum_j m_j * S_j
-  __device__ static void step(const Raw &r, int q, int rr, const uint8_t *lds, int sb, ff4 &acc) {
+  // acc (per set, columns 4q..4q+3 of row rr) += d * sum(n * sc * x) - dmin * sum_j m_j * S_j
+  template <int TS>
+  __device__ static void step(const Raw &r, int q, int rr, const uint8_t *lds, int sb, ff4 (&acc)[TS]) {
     const uint4 h = r.h;
     const int k = 16 * (q & 1);
     // get_scale_min_k4 (src/Quants.cs:321-330) for sub-blocks 2q, 2q + 1
@@ -147,7 +152,9 @@ struct FQ4K {
     const fh2 sh = {b, b}, nh = {(_Float16)(-64.f * schi), (_Float16)(-64.f * schi)};
     const uint32_t qd[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
     const uint8_t *xs = lds + (int64_t)sb * 8 * 4 * FM_NS * 16;
-    ff4 C = {0.f, 0.f, 0.f, 0.f};
+    ff4 C[TS];
+#pragma unroll
+    for (int t = 0; t < TS; t++) C[t] = ff4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int m = 0; m < 8; m++) {
       const uint32_t D = qd[m], D8 = D >> 8;
@@ -156,18 +163,24 @@ struct FQ4K {
       const fh2 p2 = __builtin_elementwise_fma(as_fh2((D & 0x00F000F0u) | 0x64006400u), sh, nh);
       const fh2 p3 = __builtin_elementwise_fma(as_fh2((D8 & 0x00F000F0u) | 0x64006400u), sh, nh);
       const fh8 bv = {p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-      const fh8 av = *reinterpret_cast<const fh8 *>(xs + (int64_t)((m * 4 + q) * FM_NS + rr) * 16);
-      C = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, C, 0, 0, 0);
+#pragma unroll
+      for (int t = 0; t < TS; t++) {
+        const fh8 av = *reinterpret_cast<const fh8 *>(xs + t * FM_SET + (int64_t)((m * 4 + q) * FM_NS + rr) * 16);
+        C[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bv, C[t], 0, 0, 0);
+      }
     }
-    const float *Ss = reinterpret_cast<const float *>(lds + FM_XBYTES) + (int64_t)sb * 2 * 4 * FM_NS;
-    ff4 Mn = {0.f, 0.f, 0.f, 0.f};
-    Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(Ss[(0 * 4 + q) * FM_NS + rr], mlo, Mn, 0, 0, 0);
-    Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(Ss[(1 * 4 + q) * FM_NS + rr], mhi, Mn, 0, 0, 0);
     const float d = half_lo(h.x), dmin = half_hi(h.x);
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      acc[i] = __builtin_fmaf(d, C[i], acc[i]);
-      acc[i] = __builtin_fmaf(-dmin, Mn[i], acc[i]);
+    for (int t = 0; t < TS; t++) {
+      const float *Ss = reinterpret_cast<const float *>(lds + t * FM_SET + FM_XBYTES) + (int64_t)sb * 2 * 4 * FM_NS;
+      ff4 Mn = {0.f, 0.f, 0.f, 0.f};
+      Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(Ss[(0 * 4 + q) * FM_NS + rr], mlo, Mn, 0, 0, 0);
+      Mn = __builtin_amdgcn_mfma_f32_16x16x4f32(Ss[(1 * 4 + q) * FM_NS + rr], mhi, Mn, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        acc[t][i] = __builtin_fmaf(d, C[t][i], acc[t][i]);
+        acc[t][i] = __builtin_fmaf(-dmin, Mn[i], acc[t][i]);
+      }
     }
   }
 };
@@ -208,11 +221,14 @@ struct FQ6K {
     r.dw = ldw4(align4_down(blk) + 52);  // d: low half (block at 0 mod 4) or high half (2 mod 4)
   }
 
-  __device__ static void step(const Raw &r, int q, int rr, const uint8_t *lds, int sb, ff4 &acc) {
+  template <int TS>
+  __device__ static void step(const Raw &r, int q, int rr, const uint8_t *lds, int sb, ff4 (&acc)[TS]) {
     const int ih = q & 1;
     const uint32_t K64 = 0x64646464u;
     const uint8_t *xs = lds + (int64_t)sb * 8 * 4 * FM_NS * 16;
-    ff4 Cl = {0.f, 0.f, 0.f, 0.f}, Ch = {0.f, 0.f, 0.f, 0.f};
+    ff4 Cl[TS], Ch[TS];
+#pragma unroll
+    for (int t = 0; t < TS; t++) Cl[t] = Ch[t] = ff4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int g = 0; g < 4; g++) {
       const uint32_t sw = r.sc.dw(g >> 1);
@@ -244,15 +260,21 @@ struct FQ6K {
         }
         const fh8 bl = {wl[0][0], wl[0][1], wl[1][0], wl[1][1], wl[2][0], wl[2][1], wl[3][0], wl[3][1]};
         const fh8 bh = {wh[0][0], wh[0][1], wh[1][0], wh[1][1], wh[2][0], wh[2][1], wh[3][0], wh[3][1]};
-        const fh8 av = *reinterpret_cast<const fh8 *>(xs + (int64_t)(((2 * g + p) * 4 + q) * FM_NS + rr) * 16);
-        Cl = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bl, Cl, 0, 0, 0);
-        Ch = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bh, Ch, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TS; t++) {
+          const fh8 av =
+              *reinterpret_cast<const fh8 *>(xs + t * FM_SET + (int64_t)(((2 * g + p) * 4 + q) * FM_NS + rr) * 16);
+          Cl[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bl, Cl[t], 0, 0, 0);
+          Ch[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, bh, Ch[t], 0, 0, 0);
+        }
       }
       __builtin_amdgcn_sched_barrier(0);  // one group's operands live at a time
     }
     const float d = half_lo(r.l1.sh ? (r.dw >> 16) : r.dw);
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(d, __builtin_fmaf(16.f, Ch[i], Cl[i]), acc[i]);
+    for (int t = 0; t < TS; t++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[t][i] = __builtin_fmaf(d, __builtin_fmaf(16.f, Ch[t][i], Cl[t][i]), acc[t][i]);
   }
 };
 
@@ -275,21 +297,22 @@ __device__ __forceinline__ void fmma_prep(const BatchArgs &a, uint8_t *lds, floa
   const int wv = threadIdx.x >> 6, u = blockIdx.y;
   const int n = a.cols - u * FM_UNIT < FM_UNIT ? a.cols - u * FM_UNIT : FM_UNIT;
   if (wv < a.T) {
-    const float iv = prep_token<C>(a.x + (int64_t)wv * a.ldx + (int64_t)u * FM_UNIT, n, wv, lds);
+    const float iv = prep_token<C>(a.x + (int64_t)wv * a.ldx + (int64_t)u * FM_UNIT, n, wv & 7, lds + (wv >> 3) * FM_SET);
     if ((threadIdx.x & 63) == 0) inv[wv] = iv;
   } else {
-    prep_zero(wv, lds);
+    prep_zero(wv & 7, lds + (wv >> 3) * FM_SET);
   }
 }
 
 // One workgroup's work: the tokens' x parts of its unit into LDS, then the tiles of one matrix
-// (pair): wave wv takes tiles wgx * 8 + wv, + nwg * 8, .... The unit's items (super-block b,
+// (pair): wave wv of its W takes tiles wgx + wv * nwg, + nwg * W, ...: where a matrix has fewer tiles than
+// waves, every workgroup gets some. The unit's items (super-block b,
 // matrix m, in that order) are computed with the loads of the next PF items in flight; the
 // first tile's first loads are issued before the x parts are prepared.
-template <class C, int NM>
+template <class C, int NM, int TS>
 __device__ __forceinline__ void fmma_body(const BatchArgs &a, const BatchMat &M, int wgx, int nwg, uint8_t *lds,
                                           float *inv) {
-  constexpr int PF = fmma_ahead<C, NM>();
+  constexpr int PF = fmma_ahead<C, NM>(), W = fm_waves(TS);
   // a ring of PF + 1 load buffers; a loop body of K items keeps every buffer's role and every
   // item's matrix fixed at compile time. Past the last item the last one is re-read (valid
   // memory, unused), so every load is issued and the load counters' waits stay exact.
@@ -298,7 +321,7 @@ __device__ __forceinline__ void fmma_body(const BatchArgs &a, const BatchMat &M,
   const int q = lane >> 4, rr = lane & 15, u = blockIdx.y;
   const int rem = (a.cols - u * FM_UNIT) / 256;
   const int nsb = rem < 8 ? rem : 8, NI = nsb * NM;
-  const int ntiles = (M.rows + 15) / 16, first = wgx * FM_WAVES + wv;
+  const int ntiles = (M.rows + 15) / 16, first = wgx + wv * nwg;
   const uint8_t *wr[NM];
   auto rows_of = [&](int tile) {
     const int row = min(tile * 16 + rr, M.rows - 1);
@@ -319,14 +342,16 @@ __device__ __forceinline__ void fmma_body(const BatchArgs &a, const BatchMat &M,
   }
   fmma_prep<C>(a, lds, inv);
   __syncthreads();
-  for (int tile = first; tile < ntiles; tile += nwg * FM_WAVES) {
+  for (int tile = first; tile < ntiles; tile += nwg * W) {
     if (tile != first) {
       rows_of(tile);
       preload();
     }
-    ff4 acc[NM];
+    ff4 acc[NM][TS];
 #pragma unroll
-    for (int m = 0; m < NM; m++) acc[m] = ff4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < NM; m++)
+#pragma unroll
+      for (int t = 0; t < TS; t++) acc[m][t] = ff4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
     for (int base = 0; base < NI; base += K) {
 #pragma unroll
@@ -335,18 +360,21 @@ __device__ __forceinline__ void fmma_body(const BatchArgs &a, const BatchMat &M,
         if (i < NI) {  // uniform
           const int j = i + PF < NI ? i + PF : NI - 1;
           C::load(wr[(k + PF) % NM] + (int64_t)(j / NM) * C::BYTES, q, rg[(k + PF) % (PF + 1)]);
-          C::step(rg[k % (PF + 1)], q, rr, lds, i / NM, acc[k % NM]);
+          C::template step<TS>(rg[k % (PF + 1)], q, rr, lds, i / NM, acc[k % NM]);
         }
       }
     }
     const int r = tile * 16 + rr;
     if (r < M.rows) {
-      const int t0 = 2 * q, t1 = 2 * q + 1;
 #pragma unroll
-      for (int m = 0; m < NM; m++) {
-        float *pm = M.part + (int64_t)m * a.T * M.rows * a.u;
-        if (t0 < a.T) pm[((int64_t)t0 * M.rows + r) * a.u + u] = (acc[m][0] + acc[m][1]) * inv[t0];
-        if (t1 < a.T) pm[((int64_t)t1 * M.rows + r) * a.u + u] = (acc[m][2] + acc[m][3]) * inv[t1];
+      for (int s = 0; s < TS; s++) {
+        const int t0 = 8 * s + 2 * q, t1 = t0 + 1;
+#pragma unroll
+        for (int m = 0; m < NM; m++) {
+          float *pm = M.part + (int64_t)m * a.T * M.rows * a.u;
+          if (t0 < a.T) pm[((int64_t)t0 * M.rows + r) * a.u + u] = (acc[m][s][0] + acc[m][s][1]) * inv[t0];
+          if (t1 < a.T) pm[((int64_t)t1 * M.rows + r) * a.u + u] = (acc[m][s][2] + acc[m][s][3]) * inv[t1];
+        }
       }
     }
   }
@@ -354,27 +382,33 @@ __device__ __forceinline__ void fmma_body(const BatchArgs &a, const BatchMat &M,
 
 // KINDS: the formats present (1: Q4_K, 2: Q6_K, 3: both, the fused q/k/v of a Q4_K_M layer);
 // a kernel holds only the codecs it needs, so each stays within its register budget.
-template <int NM, int KINDS>
-__global__ __launch_bounds__(64 * FM_WAVES) __attribute__((amdgpu_waves_per_eu(4))) void fmma_kernel(BatchArgs a) {
-  __shared__ float inv[FM_WAVES];
+template <int NM, int KINDS, int TS>
+__global__ __launch_bounds__(64 * fm_waves(TS)) __attribute__((amdgpu_waves_per_eu(4))) void fmma_kernel(BatchArgs a) {
+  __shared__ float inv[fm_waves(TS)];
   uint8_t *lds = wl_dyn_lds;
   const int mi = batch_mat(a);
   const BatchMat &M = a.m[mi];
   const int wgx = (int)blockIdx.x - M.wg_begin, nwg = batch_nwg(a, mi);
   const bool q4 = KINDS == 1 || (KINDS == 3 && M.type == 12);  // uniform over the workgroup
   if constexpr (KINDS & 1)
-    if (q4) fmma_body<FQ4K, NM>(a, M, wgx, nwg, lds, inv);
+    if (q4) fmma_body<FQ4K, NM, TS>(a, M, wgx, nwg, lds, inv);
   if constexpr ((KINDS & 2) != 0)
-    if (!q4) fmma_body<FQ6K, NM>(a, M, wgx, nwg, lds, inv);
+    if (!q4) fmma_body<FQ6K, NM, TS>(a, M, wgx, nwg, lds, inv);
+}
+
+template <int NM, int KINDS, int TS>
+static hipError_t fmma_launch_ts(const BatchArgs &a, int gx, hipStream_t st) {
+  static bool raised = false;
+  const size_t smem = (size_t)FM_SET * TS;
+  hipError_t e = raise_lds(&fmma_kernel<NM, KINDS, TS>, smem, raised);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((fmma_kernel<NM, KINDS, TS>), dim3(gx, a.u), dim3(64 * fm_waves(TS)), smem, st, a);
+  return hipGetLastError();
 }
 
 template <int NM, int KINDS>
-static hipError_t fmma_launch(const BatchArgs &a, int gx, size_t smem, hipStream_t st) {
-  static bool raised = false;
-  hipError_t e = raise_lds(&fmma_kernel<NM, KINDS>, smem, raised);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((fmma_kernel<NM, KINDS>), dim3(gx, a.u), dim3(64 * FM_WAVES), smem, st, a);
-  return hipGetLastError();
+static hipError_t fmma_launch(const BatchArgs &a, int gx, hipStream_t st) {
+  return a.T > 8 ? fmma_launch_ts<NM, KINDS, 2>(a, gx, st) : fmma_launch_ts<NM, KINDS, 1>(a, gx, st);
 }
 
 // ------------------------------------------------------------------------------------ host
@@ -399,7 +433,7 @@ int64_t fmma_scratch_floats(const GemvMat *mats, int nmat, int nm, int cols, int
 
 hipError_t fmma_run(const GemvMat *mats, int nmat, int nm, const float *x, int ldx, int cols, int T,
                     float *scratch, int num_cu, hipStream_t st) {
-  if (!fmma_applies(mats, nmat, nm, cols) || T < 1 || T > 8 || !scratch || num_cu < 1) return hipErrorInvalidValue;
+  if (!fmma_applies(mats, nmat, nm, cols) || T < 1 || T > FMMA_MAX_T || !scratch || num_cu < 1) return hipErrorInvalidValue;
   BatchArgs a{};
   a.u = fmma_units(cols);
   a.S = 1;
@@ -409,13 +443,14 @@ hipError_t fmma_run(const GemvMat *mats, int nmat, int nm, const float *x, int l
   a.x = x;
   a.ldx = ldx;
   a.T = T;
-  // one round of two resident workgroups per CU: tiles per wave so that the grid covers every
-  // (matrix, unit) tile once, then workgroups per matrix in proportion to its tiles
+  // One round of 16 resident waves per CU (two workgroups, or one of 16 waves), the workgroups shared
+  // out by the matrices' tiles: tiles of few rows go to all CUs, a few waves of each (grouped eight to
+  // a workgroup, 8B q/k/v at 8 tokens used 96 workgroups of 512 and took 18.8 us).
+  const int W = fm_waves(T > 8 ? 2 : 1);
   int64_t tiles = 0;
   for (int i = 0; i < nmat; i++) tiles += (mats[i].rows + 15) / 16;
-  const int64_t waves = (int64_t)num_cu * 2 * FM_WAVES;
-  int64_t tpw = (tiles * a.u + waves - 1) / waves;
-  if (tpw < 1) tpw = 1;
+  int64_t want = (int64_t)num_cu * 16 / W / a.u;
+  if (want < 1) want = 1;
   float *part = scratch;
   int gx = 0;
   for (int i = 0; i < nmat; i++) {
@@ -423,16 +458,16 @@ hipError_t fmma_run(const GemvMat *mats, int nmat, int nm, const float *x, int l
     a.m[i] = BatchMat{m.w, m.w2, m.row_bytes, part, m.y, m.ldy, m.rows, m.type, gx, m.add, m.rs};
     part += (int64_t)a.u * nm * T * m.rows;
     const int64_t t = (m.rows + 15) / 16;
-    gx += (int)((t + FM_WAVES * tpw - 1) / (FM_WAVES * tpw));
+    int64_t n = (want * t + tiles - 1) / tiles;
+    gx += (int)(n > t ? t : n);
   }
-  const size_t smem = FM_XBYTES + FM_SBYTES;
   int kinds = 0;
   for (int i = 0; i < nmat; i++) kinds |= mats[i].type == 12 ? 1 : 2;
   hipError_t e;
-  if (nm == 2) e = kinds == 1 ? fmma_launch<2, 1>(a, gx, smem, st) : fmma_launch<2, 2>(a, gx, smem, st);
-  else if (kinds == 1) e = fmma_launch<1, 1>(a, gx, smem, st);
-  else if (kinds == 2) e = fmma_launch<1, 2>(a, gx, smem, st);
-  else e = fmma_launch<1, 3>(a, gx, smem, st);
+  if (nm == 2) e = kinds == 1 ? fmma_launch<2, 1>(a, gx, st) : fmma_launch<2, 2>(a, gx, st);
+  else if (kinds == 1) e = fmma_launch<1, 1>(a, gx, st);
+  else if (kinds == 2) e = fmma_launch<1, 2>(a, gx, st);
+  else e = fmma_launch<1, 3>(a, gx, st);
   if (e != hipSuccess) return e;
   return nm == 1 ? launch_batch_combine<1>(a, st) : launch_batch_combine<2>(a, st);
 }

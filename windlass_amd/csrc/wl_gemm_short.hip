@@ -13,8 +13,8 @@
 // Lane (q = l / 16, rr = l % 16) of a wave holds quarter q of row rr's 256 columns, and chunk m =
 // 2 g + p is v_mfma_f32_16x16x32_bf16 with the lane's values 8 p .. 8 p + 7 of its run g of 16. Which
 // columns a quarter is follows the format, so that no lane loads a byte that another uses and every
-// field is one load of up to 16 bytes (a load costs the texture unit a cycle per row and lane; the
-// 34-byte blocks of Q8_0 took 6 a run as aligned dword windows, 49 us of 14336 x 4096 at 9 tokens):
+// field is a few loads of 16 bytes (in order 0 the 34-byte blocks of Q8_0 took 6 loads a run, 49 us of
+// 14336 x 4096 at 9 tokens):
 //   order 0 (Q4_K, Q5_K, Q6_K): q = 2 hh + ih is columns 128 hh + 32 g + 16 ih + (0..15)
 //   order 1 (Q8_0, IQ4_XS):     64 q + 16 g + (0..15)
 // x comes in the same order (wl_frag.h), 1 KB contiguous per chunk and 16 tokens, from L2 into
@@ -132,29 +132,50 @@ __device__ __forceinline__ uint4 scaled_chunk(float s, uint32_t a, uint32_t b) {
                     pk_bf16(s * sb(b, 0), s * sb(b, 1)), pk_bf16(s * sb(b, 2), s * sb(b, 3)));
 }
 
+// Blocks at 2-byte alignment come as aligned dword windows (a load at 2-byte alignment is slower than
+// the window's extra dword: Q6_K 14336 x 4096 at 9 tokens 33 us with them).
 struct SQ6K {
   static constexpr int BYTES = 210;
-  struct Raw { uint4 l0, l1, qh; uint2 sc; uint32_t d; };
+  // every field offset is a multiple of 4: the fields share the block's misalignment
+  struct Raw { uint32_t l0[5], l1[5], qh[5], sc[3], dw, sh; };
   struct Scale { float ds[4]; };
-  __device__ static void load(const uint8_t *b, int q, Raw &r) {
+  __device__ static void window(gu32 *a, uint32_t (&o)[5]) {
+    const u32x4a4_t v = *reinterpret_cast<gu32x4 *>(a);
+    o[0] = v.x;
+    o[1] = v.y;
+    o[2] = v.z;
+    o[3] = v.w;
+    o[4] = ldw4(a + 4);
+  }
+  __device__ static void load(const uint8_t *blk, int q, Raw &r) {
     const int hh = q >> 1, ih = q & 1;
-    r.l0 = ldw16_a2(b + 64 * hh + 16 * ih);
-    r.l1 = ldw16_a2(b + 64 * hh + 32 + 16 * ih);
-    r.qh = ldw16_a2(b + 128 + 32 * hh + 16 * ih);
-    r.sc = ldw8_a2(b + 192 + 8 * hh);
-    r.d = ldw2(b + 208);
+    gu32 *a = align4_down(blk);
+    r.sh = misalign4(blk) * 8;
+    window(a + 16 * hh + 4 * ih, r.l0);
+    window(a + 16 * hh + 8 + 4 * ih, r.l1);
+    window(a + 32 + 8 * hh + 4 * ih, r.qh);
+    ldw12(a + 48 + 2 * hh, r.sc);
+    r.dw = ldw4(a + 52);
   }
   __device__ static Scale scale(const Raw &r, int q) {
-    const float d = half_lo(r.d);
-    const uint32_t a = r.sc.x >> (8 * (q & 1)), b = r.sc.y >> (8 * (q & 1));  // scale bytes 2g + ih of the half's 8
-    return Scale{{d * sb(a, 0), d * sb(a, 2), d * sb(b, 0), d * sb(b, 2)}};
+    const float d = half_lo(r.dw >> r.sh);
+    Scale s;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {  // scale bytes 2g + ih of the half's 8
+      const uint32_t w = __builtin_amdgcn_alignbit(r.sc[i + 1], r.sc[i], r.sh) >> (8 * (q & 1));
+      s.ds[2 * i] = d * sb(w, 0);
+      s.ds[2 * i + 1] = d * sb(w, 2);
+    }
+    return s;
   }
   __device__ static uint4 frag(const Raw &r, const Scale &s, int, int m) {
     const int g = m >> 1, p = m & 1;
     uint32_t w[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {  // src/Quants.cs:381-392
-      const uint32_t L = dw_at((g & 1) ? r.l1 : r.l0, 2 * p + i), H = dw_at(r.qh, 2 * p + i);
+      const uint32_t *ql = (g & 1) ? r.l1 : r.l0;
+      const uint32_t L = __builtin_amdgcn_alignbit(ql[2 * p + i + 1], ql[2 * p + i], r.sh);
+      const uint32_t H = __builtin_amdgcn_alignbit(r.qh[2 * p + i + 1], r.qh[2 * p + i], r.sh);
       const uint32_t v = ((L >> (4 * (g >> 1))) & 0x0F0F0F0Fu) | (((H >> (2 * g)) & 0x03030303u) << 4);
       // q - 32 per byte (0 <= q < 64): bit 7 set keeps the borrow inside its byte
       w[i] = ((v | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
@@ -163,24 +184,36 @@ struct SQ6K {
   }
 };
 
-// Quarter q is 34-byte blocks 2q and 2q + 1 of the eight, runs 2 and 3 the second's.
+// Quarter q is 34-byte blocks 2q and 2q + 1 of the eight, 68 contiguous bytes: d f16 | int8[32] twice.
 struct SQ80 {
   static constexpr int BYTES = 272;
-  struct Raw { uint4 v[4]; uint32_t d[2]; };
+  struct Raw { uint32_t w[18], sh; };  // the aligned dwords around the 68 bytes
   struct Scale { float d[2]; };
   __device__ static void load(const uint8_t *blk, int q, Raw &r) {
+    const uint8_t *b = blk + 68 * q;
+    gu32 *a = align4_down(b);
+    r.sh = misalign4(b) * 8;
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-      const uint8_t *b = blk + 68 * q + 34 * i;
-      r.d[i] = ldw2(b);
-      r.v[2 * i] = ldw16_a2(b + 2);
-      r.v[2 * i + 1] = ldw16_a2(b + 18);
+    for (int i = 0; i < 4; i++) {
+      const u32x4a4_t v = *reinterpret_cast<gu32x4 *>(a + 4 * i);
+      r.w[4 * i] = v.x;
+      r.w[4 * i + 1] = v.y;
+      r.w[4 * i + 2] = v.z;
+      r.w[4 * i + 3] = v.w;
     }
+    r.w[16] = ldw4(a + 16);
+    r.w[17] = ldw4(a + 17);
   }
-  __device__ static Scale scale(const Raw &r, int) { return Scale{{half_lo(r.d[0]), half_lo(r.d[1])}}; }
+  // dword i of the 68 bytes; the quants start at byte 2 (first block) and 36
+  __device__ static uint32_t dw(const Raw &r, int i) { return __builtin_amdgcn_alignbit(r.w[i + 1], r.w[i], r.sh); }
+  __device__ static Scale scale(const Raw &r, int) { return Scale{{half_lo(dw(r, 0)), half_hi(dw(r, 8))}}; }
   __device__ static uint4 frag(const Raw &r, const Scale &s, int, int m) {  // src/Quants.cs:257
-    const int g = m >> 1, p = m & 1;
-    return scaled_chunk(s.d[g >> 1], dw_at(r.v[g], 2 * p), dw_at(r.v[g], 2 * p + 1));
+    const int g = m >> 1, p = m & 1, i = 4 * (g & 1) + 2 * p;
+    uint32_t w[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+      w[k] = g < 2 ? __builtin_amdgcn_alignbit(dw(r, i + k + 1), dw(r, i + k), 16) : dw(r, 9 + i + k);
+    return scaled_chunk(s.d[g >> 1], w[0], w[1]);
   }
 };
 
