@@ -788,10 +788,10 @@ extern "C" int wl_matmul_add_dev(wl_ctx *c, const wl_weight *w, int32_t expert, 
   return WL_OK;
 }
 
-// A small host product's x and y pass through the context's pinned memory, moved by a kernel: a copy of
+// A small host product's x and y (up to 1 MB each) pass through the context's pinned memory, moved by a kernel: a copy of
 // pageable memory is staged, queued and waited for by the runtime (Q8_0 4096 x 4096 at one token 33 us,
 // of which the GPU worked 11). Larger arrays keep the runtime's copies, whose cost is the transfer.
-static constexpr size_t kIoBytes = (size_t)256 << 10;
+static constexpr size_t kIoBytes = (size_t)1 << 20;
 
 static __global__ __launch_bounds__(256) void io_copy_kernel(const uint32_t *__restrict__ src, uint32_t *__restrict__ dst,
                                                              int n) {
