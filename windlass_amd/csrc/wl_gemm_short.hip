@@ -7,7 +7,7 @@
 //
 // A workgroup owns 16 R rows and splits K over its KW waves, whose sums meet in LDS at the end in
 // wave order: the launch fills the device without partial planes in memory and a launch to add
-// them. The split depends on the columns and the tokens alone, so a matrix gives the same bits
+// them. The split depends on the columns alone, so a matrix gives the same bits
 // alone, beside others in one launch, or as gate or up.
 //
 // Lane (q = l / 16, rr = l % 16) of a wave holds quarter q of row rr's 256 columns, and chunk m =
@@ -257,6 +257,12 @@ struct ShortArgs {
   int hord;
 };
 
+// Token tiles whose waves' sums meet in LDS at a time: a result per thread.
+constexpr int short_round(int kw, int r, int nt) {
+  const int n = kw * 64 / (256 * r) < 1 ? 1 : kw * 64 / (256 * r);
+  return n < nt ? n : nt;
+}
+
 // One row group of 16 R rows (PAIR: 16 of gate, 16 of up) by NT token tiles.
 template <class C, int R, int NT, int KW, bool PAIR>
 __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &mat, int row0, float *red) {
@@ -318,7 +324,7 @@ __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &m
   }
   // the waves' sums in wave order, TR token tiles at a time: lane holds rows 4 q .. 4 q + 3 of
   // token rr of a tile
-  constexpr int TR = KW * 64 / (256 * R) < NT ? KW * 64 / (256 * R) : NT;
+  constexpr int TR = short_round(KW, R, NT);
   sf4 *red4 = reinterpret_cast<sf4 *>(red);
 #pragma unroll
   for (int t1 = 0; t1 < NT; t1 += TR) {
@@ -331,8 +337,8 @@ __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &m
       }
     __syncthreads();
     if constexpr (PAIR) {
-      if (tid < TR * 256) {
-        const int t = tid >> 8, e = tid & 255, tok = 16 * (t1 + t) + (e >> 4);
+      for (int el = tid; el < TR * 256; el += KW * 64) {
+        const int t = el >> 8, e = el & 255, tok = 16 * (t1 + t) + (e >> 4);
         float g = 0.f, u = 0.f;
 #pragma unroll
         for (int w = 0; w < KW; w++) {
@@ -345,15 +351,17 @@ __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &m
           a.hf[frag_at(tok, row & ~7, mat.rows, a.hord) * 8 + (row & 7)] = __builtin_bit_cast(uint16_t, h);
         }
       }
-    } else if (tid < TR * R * 256) {
-      const int t = tid / (256 * R), r = (tid >> 8) % R, e = tid & 255, tok = 16 * (t1 + t) + (e >> 4);
-      float s = 0.f;
+    } else {
+      for (int el = tid; el < TR * R * 256; el += KW * 64) {
+        const int t = el / (256 * R), r = (el >> 8) % R, e = el & 255, tok = 16 * (t1 + t) + (e >> 4);
+        float s = 0.f;
 #pragma unroll
-      for (int w = 0; w < KW; w++) s += red[((w * TR + t) * R + r) * 256 + e];
-      const int row = row0 + 16 * r + (e & 15);
-      if (t1 + t < NT && tok < a.T && row < mat.rows) {
-        float *yp = mat.y + (int64_t)tok * mat.ldy + row;
-        *yp = a.add ? add_scaled(*yp, s, a.rs) : s;
+        for (int w = 0; w < KW; w++) s += red[((w * TR + t) * R + r) * 256 + e];
+        const int row = row0 + 16 * r + (e & 15);
+        if (t1 + t < NT && tok < a.T && row < mat.rows) {
+          float *yp = mat.y + (int64_t)tok * mat.ldy + row;
+          *yp = a.add ? add_scaled(*yp, s, a.rs) : s;
+        }
       }
     }
   }
@@ -361,7 +369,7 @@ __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &m
 
 template <int R, int NT, int KW, bool PAIR>
 __global__ __launch_bounds__(64 * KW) void short_kernel(ShortArgs a) {
-  __shared__ float red[KW * KW * 64];
+  __shared__ float red[KW * short_round(KW, R, NT) * R * 256];
   const int rg = blockIdx.x;
   int k = 0;
   if constexpr (!PAIR) {
@@ -400,20 +408,29 @@ hipError_t go(const ShortArgs &a, int groups, hipStream_t st) {
   return hipGetLastError();
 }
 
-constexpr int kWaves = 8;    // that share a row's columns
 constexpr int kShortT = 128;  // tokens at most: 8 tiles' accumulators
 
+template <int R, int KW, bool PAIR>
+hipError_t dispatch_kw(const ShortArgs &a, int groups, hipStream_t st) {
+  switch (a.tiles) {
+    case 1: return go<R, 1, KW, PAIR>(a, groups, st);
+    case 2: return go<R, 2, KW, PAIR>(a, groups, st);
+    case 3: return go<R, 3, KW, PAIR>(a, groups, st);
+    case 4: return go<R, 4, KW, PAIR>(a, groups, st);
+    case 5:
+    case 6: return go<R, 6, KW, PAIR>(a, groups, st);
+    default: return go<R, 8, KW, PAIR>(a, groups, st);
+  }
+}
+
+// Waves that share a row's columns: four, whose longer walks pay the first and last memory round trip
+// once for more blocks, or eight for rows past 10,240 columns, which are most of the time of matrices
+// of few rows (45 tokens: Q4_K 14336 x 4096 25.4 us with four and 28.7 with eight, 28672 x 8192 76.6 and
+// 85.1, 4096 x 4096 12.1 and 11.5, 4096 x 14336 31.5 and 30.2; at 9 tokens 22.4 and 19.7). By the columns
+// alone, so that a matrix has the same bits in every launch.
 template <int R, bool PAIR>
 hipError_t dispatch(const ShortArgs &a, int groups, hipStream_t st) {
-  switch (a.tiles) {
-    case 1: return go<R, 1, kWaves, PAIR>(a, groups, st);
-    case 2: return go<R, 2, kWaves, PAIR>(a, groups, st);
-    case 3: return go<R, 3, kWaves, PAIR>(a, groups, st);
-    case 4: return go<R, 4, kWaves, PAIR>(a, groups, st);
-    case 5:
-    case 6: return go<R, 6, kWaves, PAIR>(a, groups, st);
-    default: return go<R, 8, kWaves, PAIR>(a, groups, st);
-  }
+  return a.nblk > 40 ? dispatch_kw<R, 8, PAIR>(a, groups, st) : dispatch_kw<R, 4, PAIR>(a, groups, st);
 }
 
 ShortArgs args_of(int cols, const void *xf, int T) {
@@ -453,7 +470,8 @@ hipError_t short_matmul_launch(const ShortMat *mats, int n, int cols, const void
     rows += mats[i].rows;
   }
   // 32 rows a workgroup read x half as often; 16 where those would leave CUs without a workgroup
-  // (Q4_K, 45 tokens: 14336 x 4096 32.7 us with 16 rows and 28.6 with 32; 4096 x 4096 11.8 and 14.4)
+  // (Q4_K, 45 tokens, eight waves: 14336 x 4096 32.7 us with 16 rows and 28.6 with 32; 4096 x 4096 11.8
+  // and 14.4)
   const int R = rows / 32 >= num_cu ? 2 : 1;
   int groups = 0;
   for (int i = 0; i < n; i++) {
