@@ -137,16 +137,11 @@ __device__ __forceinline__ uint32_t ldw4(gu32 *p) {
 }
 
 // Weight fields at 2-byte alignment (34- and 210-byte blocks), one load each: the hardware takes
-// such addresses.
+// such addresses, more slowly than aligned ones.
 typedef uint32_t u32x4a2_t __attribute__((ext_vector_type(4), aligned(2)));
-typedef uint32_t u32x2a2_t __attribute__((ext_vector_type(2), aligned(2)));
 __device__ __forceinline__ uint4 ldw16_a2(const uint8_t *p) {
   const u32x4a2_t v = *reinterpret_cast<const u32x4a2_t *>(p);
   return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint2 ldw8_a2(const uint8_t *p) {
-  const u32x2a2_t v = *reinterpret_cast<const u32x2a2_t *>(p);
-  return make_uint2(v.x, v.y);
 }
 __device__ __forceinline__ uint32_t ldw2(const uint8_t *p) { return *reinterpret_cast<const uint16_t *>(p); }
 

@@ -17,7 +17,8 @@
 //     registers, one step ahead.
 // Formats other than Q4_K and Q6_K ran on 256-token tiles staged through LDS (gemm_kernel):
 // 28672 x 8192 at 512 tokens Q8_0 553 -> 239 us, IQ4_XS 531 -> 216, Q5_K 528 -> 219. Matrices that
-// share x are one launch: a 70B layer's q, k and v at 512 tokens 159 us in three, 90 together.
+// share x are one launch: a 70B layer's q, k and v at 512 tokens 160 us in three with
+// their sums, 110 together.
 // LDS traffic per step is the decoded tile written once and read by four waves (40 KB) against
 // 8 JJ MFMA per wave, and one barrier per step separates a buffer's writes
 // from its reads. v_mfma_f32_32x32x16_bf16 issues at about 1.9 PFLOP/s on a whole MI355X where
@@ -225,7 +226,9 @@ __device__ __forceinline__ float signed_value(const TSigned &o) {
   return o.d * (float)(int8_t)(o.v[I / 4] >> (8 * (I % 4)));
 }
 
-// Q8_0: eight blocks of 34 B, d f16 | int8[32] (src/Quants.cs:251-259), at 2-byte alignment.
+// Q8_0: eight blocks of 34 B, d f16 | int8[32] (src/Quants.cs:251-259), at 2-byte alignment: loads at that
+// alignment, since here each load and shift takes a product's slot (as aligned dword windows 14336 x 4096
+// at 200 tokens took 65.0 us against 60.5).
 struct TQ80 {
   static constexpr int BYTES = 272, NPREP = 2;
   struct Raw { uint4 q[4]; uint32_t d[4]; };
