@@ -50,6 +50,49 @@ def test_long_bars(ctx, t, rows, cols, T):
     test_bars(ctx, t, rows, cols, T)
 
 
+def dev_rows(ctx, w, x, T, rows, pick):
+    """Rows `pick` of W x for x [T][cols] in device memory."""
+    y = torch.full((T, rows), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    check(load().wl_matmul_dev(ctx.handle, w.handle, -1, P(x), T, P(y)))
+    ctx.sync()
+    return y[pick].cpu().numpy()
+
+
+# x of 2^31 values and a little more: its bf16 pieces pass 2 GiB at token 37,449 and 4 GiB at 74,898
+def test_prompt_past_4_gib_of_pieces(ctx):
+    rows, cols, T = 37, 28672, 75000
+    x = torch.empty((T, cols), device="cuda")
+    x.normal_(generator=torch.Generator(device="cuda").manual_seed(1))
+    pick = [0, 37440, 37448, 37449, 60000, T - 150, T - 120, T - 1]
+    xs = x[pick].cpu().numpy()
+    for t in TYPES:
+        data = blocks(t, rows, cols, seed=int(t))
+        w = ctx.upload(t, data, rows, cols)
+        tol_check(dev_rows(ctx, w, x, T, rows, pick), bf16_round(xs), bf16_round(decoded(t, data, rows, cols)), rel=1e-5,
+                  what=t.name)
+        w.free()
+
+
+# one block of columns more than the long prompts' kernel takes: x zero but for the ends of the row
+# and of the first half, so that the fp32 sums stay as short as elsewhere
+def test_prompt_past_the_widest_rows(ctx):
+    rows, cols, T = 3, (1 << 22) + 256, 129
+    x = torch.zeros((T, cols), device="cuda")
+    at = [slice(0, 512), slice(cols // 2 - 300, cols // 2 + 300), slice(cols - 512, cols)]
+    g = torch.Generator(device="cuda").manual_seed(2)
+    for a in at:
+        x[:, a].normal_(generator=g)
+    pick = [0, 31, 127, 128]
+    part = lambda v: bf16_round(np.concatenate([v[:, a] for a in at], 1))  # noqa: E731
+    xs = part(x[pick].cpu().numpy())
+    for t in TYPES:
+        data = blocks(t, rows, cols, seed=int(t))
+        w = ctx.upload(t, data, rows, cols)
+        tol_check(dev_rows(ctx, w, x, T, rows, pick), xs, part(decoded(t, data, rows, cols)), rel=1e-5, what=t.name)
+        w.free()
+
+
 def P(t):
     return ctypes.c_void_p(t.data_ptr())
 

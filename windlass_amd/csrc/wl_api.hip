@@ -649,7 +649,7 @@ static int intdot_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int
 // Prompts over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows: 9 to 128 tokens (wl_gemm_short.h), more
 // (wl_gemm_tall.hip). x goes to bf16 pieces in the order the kernel reads, then the products.
 static bool prompt_applies(const wl_weight *w, int T) {
-  return wl::short_applies(w->type, T, w->cols) || (wl::gemm_tall_applies(w->type, T) && w->cols % 256 == 0);
+  return wl::short_applies(w->type, T, w->cols) || wl::gemm_tall_applies(w->type, T, w->cols);
 }
 
 static int prompt_order(const wl_weight *w, int T) { return T > 128 ? 2 : wl::short_order(w->type); }

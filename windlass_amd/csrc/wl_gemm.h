@@ -22,8 +22,10 @@ hipError_t gemm_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, 
 // Prompts of more than 128 tokens over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows (wl_gemm_tall.hip): x (or
 // silu(g) * u) as bf16 pieces in order 2 of wl_frag.h, then up to three matrices on them in one
 // launch (y, or y += result * rs), with tall_part_bytes of scratch, at most limit.
-bool gemm_tall_applies(int type, int T);
+bool gemm_tall_applies(int type, int T, int64_t cols);
 constexpr int TALL_MAX_MATS = 3;
+// Columns at most: a wave's four token blocks of them are 1 GiB of pieces, within 32-bit offsets.
+constexpr int64_t TALL_MAX_COLS = 1 << 22;
 struct TallMat {
   const uint8_t *w;
   int64_t row_bytes;

@@ -1,6 +1,7 @@
 // wl_gemm.hip - prefill GEMM over raw GGUF rows on the bf16 matrix cores (T > 8) for the formats
-// that the short and tall kernels (wl_gemm_short.hip, wl_gemm_tall.hip) do not hold, and for calls
-// of theirs whose operands would not fit the allocation-free entry's scratch.
+// that the short and tall kernels (wl_gemm_short.hip, wl_gemm_tall.hip) do not hold, for rows of more
+// columns than the tall kernel's offsets reach (TALL_MAX_COLS), and for calls of theirs whose operands
+// would not fit the allocation-free entry's scratch.
 //
 // Replaces the CPU path's batch branch of Transformer.MatMul (src/Transformer.cs:526-536):
 // decode a tile of weight rows, then FastMath.Block (src/FastMath.cs:216-264) multiplies it by

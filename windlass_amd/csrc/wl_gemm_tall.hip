@@ -339,7 +339,6 @@ struct TallArgs {
   int nmat, cols, T;
   int kc;           // columns per K-chunk (whole blocks)
   const uint4 *xf;
-  int64_t xf_bytes;
   int tiles_m, tiles_n, nwg, remap;
   int add;          // y += result * rs
   float rs;
@@ -347,18 +346,18 @@ struct TallArgs {
 
 typedef uint32_t u32x4v_t __attribute__((ext_vector_type(4)));
 
-// The wave's view of x: a buffer resource over xf, the byte offset of its first fragment block,
-// and the per-lane offset of a fragment load.
+// The wave's view of x: a buffer resource over its own JJ token blocks (a resource and its offsets
+// have 32 bits; all of xf passes 4 GiB from T * cols = 2^31 on), and the per-lane offset of a
+// fragment load.
 struct XView {
   __amdgpu_buffer_rsrc_t rs;
-  int base;     // bytes: first token block * nsteps * 2048
-  int stride;   // bytes between token blocks: nsteps * 2048
+  int stride;   // bytes between token blocks: nsteps * 2048, at most 2^28 (TALL_MAX_COLS)
   int vlane;    // lane * 16
 };
 
 // Fragment (token block jj of the wave, step s, half u) into registers.
 __device__ __forceinline__ uint4 x_frag(const XView &xv, int jj, int s, int u) {
-  const u32x4v_t v = __builtin_amdgcn_raw_buffer_load_b128(xv.rs, xv.vlane + u * 1024, xv.base + jj * xv.stride + s * 2048, 0);
+  const u32x4v_t v = __builtin_amdgcn_raw_buffer_load_b128(xv.rs, xv.vlane + u * 1024, jj * xv.stride + s * 2048, 0);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
@@ -518,13 +517,13 @@ __device__ __forceinline__ void tall_body(const TallArgs &p, const TallMat &M, f
   const int ao = (lane & 31) * TLDK + 8 * (lane >> 5);
 
   // this wave's JJ token blocks from jb. Where they pass the last real block (jlast), the wave loads
-  // the JJ blocks ending at jlast instead (a load past xf's end gives zeros) and stores only its own.
+  // the JJ blocks ending at jlast instead and stores only its own (T > 128: there are JJ blocks).
   const int jlast = (p.T - 1) / 32, jb = (n0 + TWN * wv) / 32;
   const int jfirst = jb + JJ - 1 > jlast ? max(0, jlast - JJ + 1) : jb;
   XView xv;
-  xv.rs = __builtin_amdgcn_make_buffer_rsrc((void *)p.xf, (short)0, (int)p.xf_bytes, 0x00020000);
   xv.stride = nsteps * 2048;
-  xv.base = jfirst * xv.stride;
+  xv.rs = __builtin_amdgcn_make_buffer_rsrc((void *)((const uint8_t *)p.xf + (int64_t)jfirst * xv.stride), (short)0,
+                                            min(JJ, jlast + 1 - jfirst) * xv.stride, 0x00020000);
   xv.vlane = lane * 16;
   const int s0 = kb / TK;
 
@@ -687,7 +686,9 @@ TallPlan tall_plan(const TallMat *mats, int n, int cols, int T, int num_cu, int6
 
 }  // namespace
 
-bool gemm_tall_applies(int type, int T) { return T > 128 && (type == 8 || (type >= 12 && type <= 14) || type == 23); }
+bool gemm_tall_applies(int type, int T, int64_t cols) {
+  return T > 128 && (type == 8 || (type >= 12 && type <= 14) || type == 23) && cols % 256 == 0 && cols <= TALL_MAX_COLS;
+}
 
 int64_t tall_part_bytes(const TallMat *mats, int n, int cols, int T, int num_cu, int64_t limit) {
   const TallPlan pl = tall_plan(mats, n, cols, T, num_cu, limit);
@@ -710,14 +711,14 @@ hipError_t tall_silu_frag_launch(const float *g, const float *u, int T, int cols
 
 hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *xf, int T, bool add, float rs,
                               void *part, int64_t limit, int num_cu, hipStream_t st) {
-  if (n < 1 || n > TALL_MAX_MATS || cols <= 0 || cols % 256 || T < 1 || !xf) return hipErrorInvalidValue;
+  if (n < 1 || n > TALL_MAX_MATS || cols <= 0 || !xf) return hipErrorInvalidValue;
   TallArgs a{};
   int64_t tiles = 0;
   int most = 0;
   bool v4 = true;
   for (int i = 0; i < n; i++) {
     const TallMat &m = mats[i];
-    if (m.rows < 1 || !gemm_tall_applies(m.type, INT32_MAX)) return hipErrorInvalidValue;
+    if (m.rows < 1 || !gemm_tall_applies(m.type, T, cols)) return hipErrorInvalidValue;
     a.m[i] = m;
     a.tile0[i] = (int)tiles;
     tiles += (m.rows + RM - 1) / RM;
@@ -736,7 +737,6 @@ hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *
   a.T = T;
   a.kc = pl.kc;
   a.xf = (const uint4 *)xf;
-  a.xf_bytes = frag_bytes(T, cols, 2);
   a.tiles_m = (int)tiles;
   a.tiles_n = pl.tiles_n;
   a.nwg = (int)tiles * pl.tiles_n * pl.S;
