@@ -83,6 +83,29 @@ def test_error_no_larger_than_row_by_row(ctx, qs, scale):
     assert new <= max(1.05 * old, 2.0 ** -23)
 
 
+# short prompts and flat softmaxes, where an error of the probabilities is not averaged over many terms
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("T,pos0", [(16, 0), (38, 0), (109, 0), (130, 300), (751, 1847)])
+@pytest.mark.parametrize("qs", [0.1, 0.3, 1.0])
+def test_error_no_larger_on_flat_softmaxes(ctx, qs, T, pos0, hd):
+    heads, kvh, scale = 16, 4, hd ** -0.5
+    q, K, V, n = case(T, heads, kvh, hd, pos0, qs, seed=17)
+    want = ref(q, K[:n], V[:n], heads, kvh, hd, pos0, scale)
+    rms = lambda y: float(((y - want) ** 2).mean().sqrt() / (want ** 2).mean().sqrt())  # noqa: E731
+    new, old = rms(run(ctx, q, K, V, heads, kvh, hd, pos0, scale)), rms(run(ctx, q, K, V, heads, kvh, hd, pos0, scale, 8))
+    print("rms error: tiles %.3g, rows %.3g" % (new, old))
+    assert new <= 1.05 * old
+
+
+@pytest.mark.parametrize("qs", [1e9, 1e13, 1e30])
+def test_scores_past_fp32_integers(ctx, qs):
+    # scores whose last place in fp32 is many units: one key takes each row's whole weight
+    heads, kvh, hd, T, pos0 = 4, 2, 64, 40, 300
+    q, K, V, n = case(T, heads, kvh, hd, pos0, qs, seed=3)
+    got, want = run(ctx, q, K, V, heads, kvh, hd, pos0, 0.125), ref(q, K[:n], V[:n], heads, kvh, hd, pos0, 0.125)
+    assert float((got - want).abs().max()) <= 2e-6 * float(want.abs().max())
+
+
 def test_nonfinite_rows_reach_only_their_readers(ctx):
     heads, kvh, hd, T, pos0 = 4, 2, 128, 70, 40
     q, K, V, n = case(T, heads, kvh, hd, pos0, seed=9)
@@ -92,5 +115,3 @@ def test_nonfinite_rows_reach_only_their_readers(ctx):
     assert bool(same.all()) and bool((got.isinf() == old.isinf()).all())
     fin = old.isfinite()
     assert float((got - old)[fin].abs().max()) <= 4e-6 * float(old[fin].abs().max())
-
-

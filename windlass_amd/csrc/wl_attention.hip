@@ -6,14 +6,18 @@
 // exponentials cost about half as much again on the VALU. The row-by-row kernel it replaces
 // there (attention_rows_kernel: VALU products, exp in double) took 4,643 + 115 us; this one takes 343
 // (600 TFLOP/s). 64 heads, 512 tokens: 245 -> 44 us; 32 heads, 45 tokens after 300: 31 -> 17 us.
-// Root mean square error against float64 at 2,000 positions: 2.7e-7 (the row kernel 3.5e-7).
+// Root mean square error against float64: 0.4 to 0.93 of the row kernel's over 16 to 2,048 rows after 0
+// to 3,000 positions with queries of deviation 0.3 to 30 (6.6e-8 against 7.4e-8 for 38 rows with 0.3).
 //
 // Arithmetic, at fp32's precision (Attention, src/Transformer.cs:351-393): the caches' fp16 keys
 // and values are exact operands. A query row is scaled by a power of two and split into
-// hi = fp16(q f), lo = fp16(q f - hi): 22 significant bits, exact products, fp32 sums. The
-// probabilities are exp2 in fp32 against a running maximum, carried 14 binary places up so that
-// their two fp16 parts keep 22 bits down to 2^-24 of the largest; the denominator is summed in
-// fp32 per 64 positions and in double across them.
+// hi = fp16(q f), lo = fp16(q f - hi): 22 significant bits down to 2^-17 of the head's largest value,
+// 2^-40 of that value below; exact products, fp32 sums. The probabilities are exp2 in fp32 of
+// (score - running maximum) times the scale: the difference first, so that the argument's rounding
+// is relative to the argument (a maximum scaled and rounded by itself, 14 up, left 1.6e-7 in flat
+// softmaxes, and past scores of 2^26 no probability near 1). They enter the products as two fp16
+// parts of 2^14 p: 22 bits down to 2^-16 of the largest, 2^-39 of the largest below. The denominator
+// is summed in fp32 per 64 positions and in double across them.
 //
 // Layout. S^T = K Q^T puts a query in a lane column: lane l holds 16 of every 32 keys' scores of
 // query l % 32, so the maximum takes one exchange with lane l ^ 32, and the probabilities are
@@ -38,7 +42,7 @@ typedef float ff16 __attribute__((ext_vector_type(16)));
 constexpr int kAtK = 64;   // keys per step
 constexpr int kAtQ = 32;   // tokens per wave
 constexpr int kAtW = 4;    // waves per workgroup
-constexpr float kAtUp = 14.f;
+constexpr float kAtUp = 0x1p14f;  // the probabilities' factor in their fp16 parts
 
 __device__ __forceinline__ uint32_t pk_umax16(uint32_t a, uint32_t b) {
   typedef unsigned short us2 __attribute__((ext_vector_type(2)));
@@ -233,9 +237,9 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__
 #pragma unroll
       for (int i = 0; i < 16; i++) mt = fmaxf(mt, S[s][i]);
     mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float Mn = fmaxf(M, __builtin_fmaf(mt, c2, -kAtUp));
+    const float Mn = fmaxf(M, mt);
     if (__any(Mn > M)) {
-      const float al = Mn > M ? __builtin_amdgcn_exp2f(M - Mn) : 1.f;
+      const float al = Mn > M ? __builtin_amdgcn_exp2f((M - Mn) * c2) : 1.f;
       L *= (double)al;
 #pragma unroll
       for (int d = 0; d < ND; d++)
@@ -252,11 +256,11 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__
         fh8 ph, pl;
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-          const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(S[s][8 * k + i], c2, -Mu));
+          const float p = __builtin_amdgcn_exp2f((S[s][8 * k + i] - Mu) * c2);
           ts[i & 3] += p;
-          const _Float16 a = (_Float16)p;
+          const _Float16 a = (_Float16)(p * kAtUp);
           ph[i] = a;
-          pl[i] = (_Float16)(p - (float)a);
+          pl[i] = (_Float16)__builtin_fmaf(p, kAtUp, -(float)a);  // exact
         }
 #pragma unroll
         for (int d = 0; d < ND; d++) {
@@ -290,7 +294,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__
   const bool whole = chunk >= n;  // the row's only chunk
   float *op = whole ? out + (int64_t)t * ldo + (int64_t)h * HD
                     : part + (((int64_t)t * (gridDim.x * G) + h) * gridDim.y + c) * (HD + 4);
-  const double f = whole ? 1.0 / L : 1.0;
+  const double f = (whole ? 1.0 / L : 1.0) * (1.0 / kAtUp);
 #pragma unroll
   for (int d = 0; d < ND; d++)
 #pragma unroll
@@ -302,6 +306,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__
     }
   if (!whole && hf == 0) {
     op[HD] = M;
+    op[HD + 1] = c2;
     *reinterpret_cast<double *>(op + HD + 2) = L;
   }
 }
@@ -324,7 +329,7 @@ __global__ __launch_bounds__(256) void attention_tiles_combine_kernel(const floa
   float o[HD / 64] = {};
   for (int c = 0; c < nc; c++) {
     const float *rc = rec + c * (HD + 4);
-    const float w = __builtin_amdgcn_exp2f(rc[HD] - m);
+    const float w = __builtin_amdgcn_exp2f((rc[HD] - m) * rc[HD + 1]);
     L += *reinterpret_cast<const double *>(rc + HD + 2) * (double)w;
 #pragma unroll
     for (int i = 0; i < HD / 64; i++) o[i] = __builtin_fmaf(rc[lane + 64 * i], w, o[i]);
