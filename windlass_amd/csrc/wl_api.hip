@@ -1400,9 +1400,11 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
   const bool moe = L->ffn_gate_inp != nullptr;
   const bool shared = moe && L->ffn_gate_shexp;
   int64_t FF = L->ffn_gate->rows;
-  if (L->attn_q->cols != E || L->attn_q->rows != QD || L->attn_k->rows != KD || L->attn_v->rows != KD ||
-      L->attn_output->cols != QD || L->attn_output->rows != E || L->ffn_gate->cols != E || L->ffn_up->rows != FF ||
-      L->ffn_down->cols != FF || L->ffn_down->rows != E)
+  // the matrices that share x run in one launch, over the first one's columns
+  if (L->attn_q->cols != E || L->attn_k->cols != E || L->attn_v->cols != E || L->attn_q->rows != QD ||
+      L->attn_k->rows != KD || L->attn_v->rows != KD || L->attn_output->cols != QD || L->attn_output->rows != E ||
+      L->ffn_gate->cols != E || L->ffn_up->cols != E || L->ffn_up->rows != FF || L->ffn_down->cols != FF ||
+      L->ffn_down->rows != E)
     return fail(WL_E_SHAPE, "wl_layer_dev: tensor shapes do not match the layer");
   if (moe) {
     // the router's shape here; moe_dev checks the experts and expert_used
