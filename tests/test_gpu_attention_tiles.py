@@ -115,3 +115,21 @@ def test_nonfinite_rows_reach_only_their_readers(ctx):
     assert bool(same.all()) and bool((got.isinf() == old.isinf()).all())
     fin = old.isfinite()
     assert float((got - old)[fin].abs().max()) <= 4e-6 * float(old[fin].abs().max())
+
+
+def test_many_heads_of_one_kv_head(ctx):
+    # more than 65,535 groups of four (token block, head): 516 token blocks of 512 heads
+    heads, hd, T = 512, 64, 16500
+    g = torch.Generator(device="cuda").manual_seed(1)
+    q, out = torch.empty((T, heads * hd), device="cuda").normal_(generator=g), torch.empty((T, heads * hd), device="cuda")
+    K, V = (torch.randn((T, hd), device="cuda", generator=g).half() for _ in range(2))
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    torch.cuda.synchronize()
+    check(load().wl_attention_dev(ctx.handle, P(q), T, heads, 1, hd, P(K), P(V), 0, ctypes.c_float(0.125), P(out)))
+    ctx.sync()
+    for t in (0, 31, 32, 8191, T - 1):
+        got, qt, v = out[t].reshape(heads, hd).double(), q[t].reshape(heads, hd).double(), V[:t + 1].double()
+        p = torch.softmax(qt @ K[:t + 1].double().t().contiguous() * 0.125, 1)
+        # sixteen roundings of 2^-24 of the sum's size, sum p |v|: thousands of values nearly cancel here
+        worst = float(((got - p @ v).abs() / (p @ v.abs())).max())
+        assert worst <= 2.0 ** -20, (t, worst)

@@ -64,17 +64,17 @@ __device__ __forceinline__ uint32_t finite_pair(uint32_t v) {
 
 template <int HD>
 __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__restrict__ q, int64_t ldq,
-                                                                 const uint16_t *__restrict__ K,
-                                                                 const uint16_t *__restrict__ V, int kv_dim, int G,
-                                                                 int T, int pos0, float scale, int chunk,
-                                                                 float *__restrict__ part, float *__restrict__ out,
-                                                                 int64_t ldo) {
+                                                                const uint16_t *__restrict__ K,
+                                                                const uint16_t *__restrict__ V, int kv_dim, int KH,
+                                                                int G, int chunks, int nz, int T, int pos0,
+                                                                float scale, int chunk, float *__restrict__ part,
+                                                                float *__restrict__ out, int64_t ldo) {
   constexpr int NK = HD / 16, ND = HD / 32, U = HD / 8;  // key steps, value blocks, 16-byte pieces of a row
   constexpr int KS = HD + 8, VS = kAtK + 8;              // LDS row strides (halves): 16-byte reads hit every bank
   __shared__ __attribute__((aligned(16))) uint16_t ks[kAtK * KS];
   __shared__ __attribute__((aligned(16))) uint16_t vs[HD * VS];
   __shared__ int bads[2][kAtW];
-  const int kvh = blockIdx.x, c = blockIdx.y, nz = gridDim.z, r = blockIdx.z;
+  const int kvh = blockIdx.x % KH, c = blockIdx.x / KH % chunks, r = blockIdx.x / KH / chunks;
   // longest and shortest rows in turn: the workgroups that share a CU (the grid's halves) add up
   const int z = r < (nz + 1) / 2 ? nz - 1 - r : r - (nz + 1) / 2;
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256, 2) void attention_tiles_kernel(const float *__
   L += __shfl_xor(L, 32, 64);
   const bool whole = chunk >= n;  // the row's only chunk
   float *op = whole ? out + (int64_t)t * ldo + (int64_t)h * HD
-                    : part + (((int64_t)t * (gridDim.x * G) + h) * gridDim.y + c) * (HD + 4);
+                    : part + (((int64_t)t * (KH * G) + h) * chunks + c) * (HD + 4);
   const double f = (whole ? 1.0 / L : 1.0) * (1.0 / kAtUp);
 #pragma unroll
   for (int d = 0; d < ND; d++)
@@ -367,9 +367,9 @@ static hipError_t tiles_launch(const float *q, int64_t ldq, int T, const uint16_
                                hipStream_t st) {
   const int max_n = pos0 + T, chunk = tiles_chunk(T, heads, kv_heads, max_n), S = (max_n + chunk - 1) / chunk;
   const int G = heads / kv_heads, nz = ((T + kAtQ - 1) / kAtQ * G + kAtW - 1) / kAtW;
-  if (nz > 65535 || S > 65535) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(attention_tiles_kernel<HD>, dim3(kv_heads, S, nz), dim3(256), 0, st, q, ldq, K, V, kv_dim, G, T,
-                     pos0, scale, chunk, part, out, ldo);
+  // one grid dimension: the others hold 65,535 workgroups, which 512 heads of one KV head pass at 16,400 rows
+  hipLaunchKernelGGL(attention_tiles_kernel<HD>, dim3((unsigned)((int64_t)kv_heads * S * nz)), dim3(256), 0, st, q, ldq,
+                     K, V, kv_dim, kv_heads, G, S, nz, T, pos0, scale, chunk, part, out, ldo);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || S == 1) return e;
   hipLaunchKernelGGL(attention_tiles_combine_kernel<HD>, dim3((unsigned)(((int64_t)T * heads + 3) / 4)), dim3(256), 0, st,
