@@ -363,10 +363,11 @@ int wl_layer_batch_dev(wl_ctx *ctx, const wl_layer_desc *layer, float *d_x, int3
 /* ---- Allocation-free product (no counterpart in the reference) ----
  * For callers that cannot allocate device memory: code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc. The same operation and results as wl_matmul_dev (bit
- * for bit: the same kernels), but every kernel's scratch is a static per-GPU array of 32 MiB that
- * the library resolves in wl_create, so the call allocates nothing. A call that would need more
- * scratch than that (large GEMMs: T > 8 with T * cols * 2 bytes of bf16 activations near 32 MiB)
- * returns WL_E_SHAPE before anything is launched. Calls on one GPU share the array: calls that
+ * for bit: the same kernels), but every kernel's scratch is a static per-GPU array that the library
+ * resolves in wl_create, so the call allocates nothing. A call that would need more than 32 MiB of
+ * scratch (large GEMMs: T > 8 with T * cols * 2 bytes of bf16 activations near 32 MiB, or with them a
+ * split of the columns whose sums do not fit) returns WL_E_SHAPE before anything is launched (the
+ * array's other 32 MiB take the rounding of a prompt's tokens up to whole tiles). Calls on one GPU share the array: calls that
  * overlap (other streams, other contexts, other host threads) race. */
 int wl_matmul_dev_noalloc(wl_ctx *ctx, const wl_weight *w, int32_t expert, const float *d_x, int32_t T,
                           float *d_y);

@@ -55,6 +55,44 @@ def test_noalloc_equals_matmul_dev_call_after_call():
             w.free()
 
 
+# Prompts whose scratch comes near the array's: K splits whose planes would not all fit (their best has 5
+# and 2 chunks), tokens that pass 32 MiB of bf16 only once they are rounded up to 16 or 32, and a split
+# that fits beside them
+PROMPTS = [(GgmlType.Q4_K, 11294, 6400, 179), (GgmlType.Q8_0, 16406, 3584, 793), (GgmlType.Q6_K, 19108, 7424, 136),
+           (GgmlType.Q5_K, 20, 28672, 577), (GgmlType.Q8_0, 3, 985600, 17), (GgmlType.IQ4_XS, 5000, 1280, 400)]
+
+
+@pytest.mark.parametrize("t,rows,cols,T", PROMPTS, ids=lambda v: getattr(v, "name", str(v)))
+def test_noalloc_prompts_near_the_limit(t, rows, cols, T):
+    with Context(0) as ctx:
+        w = ctx.upload(t, blocks(t, rows, cols, seed=cols), rows, cols)
+        x = np.random.default_rng(T).standard_normal((T, cols), dtype=np.float32)
+        ya, yb = _both(ctx, w, x, T)
+        assert np.array_equal(ya.view(np.uint32), yb.view(np.uint32))
+        # and so does the product added into a residual of zeros
+        dx, dy = torch.from_numpy(x).to("cuda:0"), torch.zeros((T, rows), device="cuda:0")
+        torch.cuda.synchronize()
+        check(load().wl_matmul_add_dev(ctx.handle, w.handle, -1, _p(dx), T, _p(dy), ctypes.c_float(1.0)))
+        ctx.sync()
+        assert np.array_equal(dy.cpu().numpy(), ya)
+        w.free()
+
+
+@pytest.mark.parametrize("t,rows,cols,T", [(GgmlType.Q4_K, 8192, 8192, 512), (GgmlType.Q8_0, 16384, 4096, 256)],
+                         ids=lambda v: getattr(v, "name", str(v)))
+def test_noalloc_refuses_splits_it_cannot_hold(t, rows, cols, T):
+    # planes of 4 and 2 chunks, 64 and 32 MiB, without which the device would be half empty
+    with Context(0) as ctx:
+        w = ctx.upload(t, blocks(t, rows, cols, seed=1), rows, cols)
+        dx, dy = torch.ones((T, cols), device="cuda:0"), torch.zeros((T, rows), device="cuda:0")
+        torch.cuda.synchronize()
+        with pytest.raises(ShapeError, match="scratch"):
+            check(load().wl_matmul_dev_noalloc(ctx.handle, w.handle, -1, _p(dx), T, _p(dy)))
+        ctx.sync()
+        assert not dy.any()
+        w.free()
+
+
 def test_noalloc_refuses_more_scratch_than_it_has():
     with Context(0) as ctx:
         t, rows, cols, T = GgmlType.Q4_K, 256, 28672, 1024   # bf16 copy of x alone is 56 MiB

@@ -235,9 +235,11 @@ static int ensure(wl_ctx *c, int slot, size_t bytes) {
 // ---- The allocation-free entry point's scratch ----
 // One file-scope device array per GPU, held until the process ends. In host code `scratch` only
 // names the symbol: its device address on each GPU comes from hipGetSymbolAddress with that GPU
-// current (wl_create, once per device), and only that address is handed to kernels.
+// current (wl_create, once per device), and only that address is handed to kernels. A call may need
+// kStaticScratchBytes; the other half holds what rounding a prompt's tokens up to 16 or 32 adds to its
+// bf16 operands (17 tokens to 32 at most, less than as much again).
 static constexpr size_t kStaticScratchBytes = (size_t)32 << 20;
-static __device__ __align__(256) uint8_t scratch[kStaticScratchBytes];
+static __device__ __align__(256) uint8_t scratch[2 * kStaticScratchBytes];
 static constexpr int kMaxDevices = 64;
 static std::mutex g_scratch_mu;
 static void *g_scratch_ptr[kMaxDevices];
@@ -675,13 +677,18 @@ static void tall_mats(const PromptMat *m, int n, wl::TallMat *s) {
 }
 
 // Up to three products of one x (its pieces at xf, in S_XB or the static scratch), added into their
-// y times rs with add. A long prompt's chunk partials follow the pieces.
-static int64_t prompt_part_bytes(const wl_ctx *c, const PromptMat *m, int n, int T, const void *fixed) {
+// y times rs with add. A long prompt's chunk partials follow the pieces. A product by itself is split
+// in one way whatever the entry, so that the allocation-free one gives wl_matmul_dev's bits: within the
+// static scratch, beside x in bf16, where a split that fills the device fits there. Beyond it the best
+// split is kept, and the allocation-free entry refuses the call: of 196,000 drawn products of 129 to
+// 4,000 tokens 1 in 70 has a slower split than its best by this (1.14 times at the median by
+// tall_plan's prices, 1.6 at most); if every product kept to the static scratch, 1 in 13 (1.26, 7).
+static int64_t prompt_part_bytes(const wl_ctx *c, const PromptMat *m, int n, int T) {
   if (T <= 128) return 0;
   wl::TallMat s[3];
   tall_mats(m, n, s);
-  const int64_t limit = fixed ? (int64_t)(kStaticScratchBytes - prompt_bytes(m[0].w, T)) : INT64_MAX;
-  return wl::tall_part_bytes(s, n, (int)m[0].w->cols, T, c->num_cu, limit);
+  const int64_t left = (int64_t)kStaticScratchBytes - (int64_t)T * m[0].w->cols * 2;
+  return wl::tall_part_bytes(s, n, (int)m[0].w->cols, T, c->num_cu, n == 1 && left >= 0 ? left : INT64_MAX);
 }
 
 static int prompt_products(wl_ctx *c, const PromptMat *m, int n, const void *xf, int T, bool add, float rs, void *part,
@@ -703,9 +710,10 @@ static int prompt_matmul(wl_ctx *c, const wl_weight *w, const uint8_t *base, int
                          float *d_y, bool add, float rs, void *fixed) {
   const PromptMat m{w, base, (int)rows, d_y};
   const size_t xb = prompt_bytes(w, T);
-  const int64_t pb = prompt_part_bytes(c, &m, 1, T, fixed);
+  const int64_t pb = prompt_part_bytes(c, &m, 1, T);
   void *xf = nullptr;
-  if (int rc = scratch_for(c, S_XB, xb + (size_t)pb, fixed, &xf)) return rc;
+  // what the call needs is counted in its own tokens: their rounding has room of its own there
+  if (int rc = scratch_for(c, S_XB, (fixed ? (size_t)T * w->cols * 2 : xb) + (size_t)pb, fixed, &xf)) return rc;
   WL_HIP(prompt_pieces(d_x, T, (int)w->cols, prompt_order(w, T), xf, c->stream), "gemm operands");
   return prompt_products(c, &m, 1, xf, T, add, rs, (uint8_t *)xf + xb, pb);
 }
@@ -723,8 +731,7 @@ static int matmul_dev(wl_ctx *c, const wl_weight *w, int32_t expert, const float
   int64_t rows;
   operand(w, expert, &base, &rows);
   if (int_path(c, w)) return intdot_matmul(c, w, base, rows, d_x, T, d_y, fixed);
-  if (prompt_applies(w, T) && (!fixed || prompt_bytes(w, T) <= kStaticScratchBytes))
-    return prompt_matmul(c, w, base, rows, d_x, T, d_y, false, 0.f, fixed);
+  if (prompt_applies(w, T)) return prompt_matmul(c, w, base, rows, d_x, T, d_y, false, 0.f, fixed);
   if (T > 8 && wl::gemm_supports(w->type)) {
     void *xb = nullptr;
     if ((rc = scratch_for(c, S_XB, (size_t)wl::gemm_scratch_bytes(w->type, (int)rows, (int)w->cols, T, c->num_cu), fixed,
@@ -1472,7 +1479,7 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
   auto on_x = [&](const float *norm, const PromptMat *m, int n) -> int {
     const int ord = prompt_order(m[0].w, T);
     const size_t xb = prompt_bytes(m[0].w, T);
-    const int64_t pb = prompt_part_bytes(c, m, n, T, nullptr);
+    const int64_t pb = prompt_part_bytes(c, m, n, T);
     if (int r = ensure(c, S_XB, xb + (size_t)pb)) return r;
     uint8_t *xf = (uint8_t *)c->buf[S_XB];
     if (norm && wl::rms_norm_frag_applies(d_x, E, norm)) {
@@ -1560,7 +1567,7 @@ static int layer_run(wl_ctx *c, const wl_layer_desc *L, float *d_x, int32_t T, i
     const PromptMat m[2] = {{L->ffn_gate, L->ffn_gate->dev, (int)FF, g}, {L->ffn_up, L->ffn_up->dev, (int)FF, u}};
     if ((rc = on_x(L->d_ffn_norm, m, 2))) return rc;
     const size_t hb = prompt_bytes(L->ffn_down, T);
-    const int64_t pb = prompt_part_bytes(c, &dm, 1, T, nullptr);
+    const int64_t pb = prompt_part_bytes(c, &dm, 1, T);
     if ((rc = ensure(c, S_XB, hb + (size_t)pb))) return rc;
     uint8_t *hf = (uint8_t *)c->buf[S_XB];
     WL_HIP(wl::tall_silu_frag_launch(g, u, T, (int)FF, hf, c->stream), "silu");

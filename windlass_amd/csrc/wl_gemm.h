@@ -21,7 +21,8 @@ hipError_t gemm_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, 
 
 // Prompts of more than 128 tokens over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS rows (wl_gemm_tall.hip): x (or
 // silu(g) * u) as bf16 pieces in order 2 of wl_frag.h, then up to three matrices on them in one
-// launch (y, or y += result * rs), with tall_part_bytes of scratch, at most limit.
+// launch (y, or y += result * rs), with tall_part_bytes of scratch: the planes of the best K split, or,
+// where those pass `limit` and the planes of one tile a CU do not, of the best split within it.
 bool gemm_tall_applies(int type, int T, int64_t cols);
 constexpr int TALL_MAX_MATS = 3;
 // Columns at most: a wave's four token blocks of them are 1 GiB of pieces, within 32-bit offsets.
@@ -37,6 +38,6 @@ hipError_t tall_frag_launch(const float *x, int T, int cols, void *xf, hipStream
 hipError_t tall_silu_frag_launch(const float *g, const float *u, int T, int cols, void *xf, hipStream_t st);
 int64_t tall_part_bytes(const TallMat *mats, int n, int cols, int T, int num_cu, int64_t limit);
 hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *xf, int T, bool add, float rs,
-                              void *part, int64_t limit, int num_cu, hipStream_t st);
+                              void *part, int64_t part_bytes, int num_cu, hipStream_t st);
 
 }  // namespace wl

@@ -1,7 +1,6 @@
 // wl_gemm.hip - prefill GEMM over raw GGUF rows on the bf16 matrix cores (T > 8) for the formats
-// that the short and tall kernels (wl_gemm_short.hip, wl_gemm_tall.hip) do not hold, for rows of more
-// columns than the tall kernel's offsets reach (TALL_MAX_COLS), and for calls of theirs whose operands
-// would not fit the allocation-free entry's scratch.
+// that the short and tall kernels (wl_gemm_short.hip, wl_gemm_tall.hip) do not hold, and for rows of more
+// columns than the tall kernel's offsets reach (TALL_MAX_COLS).
 //
 // Replaces the CPU path's batch branch of Transformer.MatMul (src/Transformer.cs:526-536):
 // decode a tile of weight rows, then FastMath.Block (src/FastMath.cs:216-264) multiplies it by
@@ -431,7 +430,7 @@ hipError_t gemm_launch(int type, const uint8_t *w, int64_t row_bytes, int rows, 
   float *part = reinterpret_cast<float *>(reinterpret_cast<uint8_t *>(scratch) + (int64_t)T * cols * 2);
   const int S = gemm_chunks(type, rows, cols, T, num_cu);
   switch (type) {
-    // 8, 12, 13, 14 and 23 only where 16 or 32 whole tokens of bf16 pass the caller's fixed scratch
+    // 8, 12, 13, 14 and 23: rows of more than TALL_MAX_COLS columns
     case 8: return launch<GQ80>(w, row_bytes, rows, cols, xb, T, y, ldy, part, S, st);
     case 12: return launch<GQ4K>(w, row_bytes, rows, cols, xb, T, y, ldy, part, S, st);
     case 14: return launch<GQ6K>(w, row_bytes, rows, cols, xb, T, y, ldy, part, S, st);

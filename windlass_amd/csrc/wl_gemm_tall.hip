@@ -690,11 +690,27 @@ bool gemm_tall_applies(int type, int T, int64_t cols) {
   return T > 128 && (type == 8 || (type >= 12 && type <= 14) || type == 23) && cols % 256 == 0 && cols <= TALL_MAX_COLS;
 }
 
+// K-chunks (of whole blocks) that give every CU a 512-token tile; one where 7/8 of the CUs have one unsplit.
+static int fill_chunks(int64_t tiles, int nblk, int num_cu) {
+  if (tiles * 8 >= (int64_t)num_cu * 7) return 1;
+  int64_t S = (num_cu + tiles - 1) / tiles;
+  S = S < TMAXS ? S : TMAXS;
+  S = S < nblk ? S : nblk;
+  const int64_t per = (nblk + S - 1) / S;
+  return (int)((nblk + per - 1) / per);
+}
+
 int64_t tall_part_bytes(const TallMat *mats, int n, int cols, int T, int num_cu, int64_t limit) {
-  const TallPlan pl = tall_plan(mats, n, cols, T, num_cu, limit);
-  int64_t rows = 0;
-  for (int i = 0; i < n; i++) rows += mats[i].rows;
-  return pl.S > 1 ? (int64_t)pl.S * T * rows * 4 : 0;
+  int64_t rows = 0, tiles = 0;
+  for (int i = 0; i < n; i++) {
+    rows += mats[i].rows;
+    tiles += (int64_t)((mats[i].rows + RM - 1) / RM) * ((T + 511) / 512);
+  }
+  auto planes = [&](int S) { return S > 1 ? (int64_t)S * T * rows * 4 : 0; };
+  int S = tall_plan(mats, n, cols, T, num_cu, INT64_MAX).S;
+  if (planes(S) > limit && planes(fill_chunks(tiles, cols / 256, num_cu)) <= limit)
+    S = tall_plan(mats, n, cols, T, num_cu, limit).S;
+  return planes(S);
 }
 
 hipError_t tall_frag_launch(const float *x, int T, int cols, void *xf, hipStream_t st) {
@@ -710,7 +726,7 @@ hipError_t tall_silu_frag_launch(const float *g, const float *u, int T, int cols
 }
 
 hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *xf, int T, bool add, float rs,
-                              void *part, int64_t limit, int num_cu, hipStream_t st) {
+                              void *part, int64_t part_bytes, int num_cu, hipStream_t st) {
   if (n < 1 || n > TALL_MAX_MATS || cols <= 0 || !xf) return hipErrorInvalidValue;
   TallArgs a{};
   int64_t tiles = 0;
@@ -725,7 +741,7 @@ hipError_t tall_matmul_launch(const TallMat *mats, int n, int cols, const void *
     most = m.rows > most ? m.rows : most;
     v4 = v4 && m.rows % 4 == 0 && m.ldy % 4 == 0 && reinterpret_cast<uintptr_t>(m.y) % 16 == 0;
   }
-  const TallPlan pl = tall_plan(mats, n, cols, T, num_cu, limit);
+  const TallPlan pl = tall_plan(mats, n, cols, T, num_cu, part_bytes);  // tall_part_bytes' plan
   if (pl.S > 1 && !part) return hipErrorInvalidValue;
   float *pp = (float *)part;
   for (int i = 0; i < n; i++) {
