@@ -24,7 +24,7 @@ def ctx():
     c.close()
 
 
-# one block of columns and fewer than the eight waves, an odd count (rows of 2-byte formats at both
+# one block of columns and fewer than the four waves, an odd count (rows of 2-byte formats at both
 # alignments); one row, a ragged last group, and enough rows for groups of 32 (8,200 on 256 CUs)
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: t.name)
 @pytest.mark.parametrize("rows,cols", [(1, 256), (37, 1280), (8200, 768), (500, 4352)])
@@ -38,6 +38,25 @@ def test_bars(ctx, t, rows, cols, T):
     # the bars of tests/test_gpu_gemm.py: fp32 accumulation of the bf16 operands, and bf16 itself
     tol_check(y, bf16_round(x), bf16_round(wd), rel=1e-5, what="bf16 operands")
     tol_check(y, x, wd, rel=GEMM_REL, what="fp32")
+    w.free()
+
+
+# rows past 10,240 columns, which eight waves share: an odd and an even count of column blocks, a ragged last
+# group of 16 rows and of 32 (8,200 rows, where 101 of them are checked), beside 10,240 columns on four waves
+@pytest.mark.parametrize("t", TYPES, ids=lambda t: t.name)
+@pytest.mark.parametrize("rows,cols", [(37, 10240), (37, 10496), (20, 16384), (8200, 10496)])
+def test_wide_bars(ctx, t, rows, cols):
+    data = blocks(t, rows, cols, seed=rows + cols + int(t))
+    w = ctx.upload(t, data, rows, cols)
+    pick = np.arange(rows) if rows < 100 else np.r_[0:40, 4000:4021, rows - 40:rows]
+    per = len(data) // rows
+    wd = decoded(t, np.concatenate([data[r * per:r * per + per] for r in pick]), len(pick), cols)
+    wb = bf16_round(wd)
+    for T in (9, 17, 48, 64, 65, 96, 128):  # a kernel for each count of 16-token tiles
+        x = np.random.default_rng(T).standard_normal((T, cols), dtype=np.float32)
+        y = Transformer.MatMul(w, x, T)[:, pick]
+        tol_check(y, bf16_round(x), wb, rel=1e-5, what="bf16 operands, T = %d" % T)
+        tol_check(y, x, wd, rel=GEMM_REL, what="fp32, T = %d" % T)
     w.free()
 
 
@@ -102,11 +121,23 @@ def P(t):
                                          (("Q4_K", "Q8_0", "Q6_K"), "Q6_K", "IQ4_XS")])
 @pytest.mark.parametrize("T", [9, 47, 128, 200])
 def test_layer_equals_its_operations(ctx, qkv, gu, down, T):
+    layer_equals_its_operations(ctx, qkv, gu, down, T, 512)
+
+
+# gate and up over rows that eight waves share
+@pytest.mark.parametrize("qkv,gu,down", [(("Q4_K", "Q5_K", "Q6_K"), "Q4_K", "Q6_K"), (("Q8_0",) * 3, "IQ4_XS", "Q8_0"),
+                                         (("Q6_K",) * 3, "Q6_K", "Q5_K"), (("Q8_0",) * 3, "Q8_0", "Q4_K")])
+@pytest.mark.parametrize("T", [9, 31, 47, 61, 90, 128])
+def test_wide_layer_equals_its_operations(ctx, qkv, gu, down, T):
+    layer_equals_its_operations(ctx, qkv, gu, down, T, 10496)
+
+
+def layer_equals_its_operations(ctx, qkv, gu, down, T, E):
     """A prompt's layer gives the bits of its operations called one at a time (past 128 tokens q, k and v
     may split K otherwise together than alone: the last bit of a sum moves, and some bf16 and fp16
     roundings with it)."""
     L, h, rng = load(), ctx.handle, np.random.default_rng(T)
-    E, H, KH, HD, FF, pos0 = 512, 4, 2, 64, 768, 3
+    H, KH, HD, FF, pos0 = 4, 2, 64, 768, 3
     mats = {"attn_q": (qkv[0], H * HD, E), "attn_k": (qkv[1], KH * HD, E), "attn_v": (qkv[2], KH * HD, E),
             "attn_output": ("Q4_K", E, H * HD), "ffn_gate": (gu, FF, E), "ffn_up": (gu, FF, E), "ffn_down": (down, E, FF)}
     w = {n: ctx.upload(GgmlType[t], blocks(GgmlType[t], r, c, seed=i), r, c) for i, (n, (t, r, c)) in enumerate(mats.items())}
