@@ -96,3 +96,39 @@ def test_one_expert_takes_every_token(ctx):
     assert not got[4].any() and np.isnan(got[5]).all()
     for w in ws:
         w.free()
+
+
+@pytest.mark.parametrize("T", [1024, 1025, 2100])
+def test_prompts_past_one_pass(ctx, T):
+    # 1,024 tokens a pass at most: one full pass, two of 513 and 512, three of 700
+    ne, k, embd, ff = 8, 2, 256, 512
+    ws, dense = upload(ctx, 12, 14, ne, embd, ff)
+    rng = np.random.default_rng(T)
+    x, logits = rng.standard_normal((T, embd), dtype=np.float32), rng.standard_normal((T, ne), dtype=np.float32)
+    got = dev_moe(ctx, logits, k, ws, x)
+    # every token, in sets of 100 of other places
+    order = rng.permutation(T)
+    for i in range(0, T, 100):
+        sub = order[i:i + 100] if T - i >= 109 else order[-100:]
+        assert np.array_equal(dev_moe(ctx, logits[sub], k, ws, x[sub]).view(np.uint32), got[sub].view(np.uint32))
+    pick = [0, 512, 513, 699, 700, 1023, T - 1]
+    want = moe64(logits[pick], k, dense, x[pick], ne, embd, ff)
+    for i, t in enumerate(pick):
+        assert np.max(np.abs(got[t] - want[i])) <= 1e-4 * np.std(want[i]), t
+    for w in ws:
+        w.free()
+
+
+def test_nan_logits_stay_with_their_token(ctx):
+    # a NaN logit makes every probability NaN: the first k experts with NaN weights (src/Transformer.cs:313-340)
+    ne, k, embd, ff, T = 16, 4, 256, 256, 40
+    ws, _ = upload(ctx, 14, 12, ne, embd, ff)
+    rng = np.random.default_rng(3)
+    x, logits = rng.standard_normal((T, embd), dtype=np.float32), rng.standard_normal((T, ne), dtype=np.float32)
+    want = dev_moe(ctx, logits, k, ws, x)
+    logits[7, 5], logits[39] = np.nan, np.inf
+    got = dev_moe(ctx, logits, k, ws, x)
+    rest = [t for t in range(T) if t not in (7, 39)]
+    assert np.isnan(got[[7, 39]]).all() and np.array_equal(got[rest].view(np.uint32), want[rest].view(np.uint32))
+    for w in ws:
+        w.free()
