@@ -16,9 +16,8 @@ typedef _Float16 fh8 __attribute__((ext_vector_type(8)));
 typedef float ff4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ fh2 as_fh2(uint32_t u) { return __builtin_bit_cast(fh2, u); }
-__device__ __forceinline__ uint32_t as_u32(fh2 v) { return __builtin_bit_cast(uint32_t, v); }
 
-// The unit's scale: f = 2^(15 - e) for the largest finite |x| = m 2^e (m in [0.5, 1)), and 1/f;
+// A unit's scale: f = 2^(15 - e) for the largest finite |x| = m 2^e (m in [0.5, 1)), and 1/f;
 // both powers of two, clamped to the normal range. An all-zero (or non-finite) unit takes f = 1.
 __device__ __forceinline__ void unit_scale(float mx, float &f, float &inv) {
   if (!(mx > 0.f)) {
@@ -38,18 +37,19 @@ __device__ __forceinline__ void unit_scale(float mx, float &f, float &inv) {
 // Quarter q of a super-block is sub-block pair q: qs bytes 32q..32q+31, whose low nibbles are
 // values 64q + i and high nibbles 64q + 32 + i (src/Quants.cs:333-351). MFMA m takes the lane's
 // qs dword m (bytes 4m..4m+3 of the pair) as the values 64q + {4m, 4m+2, 4m+1, 4m+3} and
-// 64q + 32 + {4m, 4m+2, 4m+1, 4m+3}: each fp16 pair is (dword & mask) | 0x6400 (1024 + n or
-// 1024 + 16n) times the sub-block scale minus 1024 sc, one packed FMA, exact.
+// 64q + 32 + {4m, 4m+2, 4m+1, 4m+3}. The quants enter centred: each fp16 pair is (dword & mask) |
+// 0x6400 (1024 + n, or 1024 + 16 n), less 1032 or 1152, times the sub-block's scale (or a sixteenth
+// of it): (n - 8) sc, exact (at most 8 * 63). Per sub-block 8 d sc - dmin m is the factor of its sum of
+// x, rounded once (both products are exact in fp32).
 struct WQ4K {
   static constexpr int BYTES = 144, NF = 1;  // NF: accumulators (MFMAs) per chunk
-  static constexpr bool MINS = true;
+  static constexpr bool MINS = true, SWAP = true;
   struct Raw { uint4 h, q0, q1; };
-  struct Scale { fh2 sl, nl, sh, nh; float mlo, mhi; };
+  struct Scale { fh2 sl, sh; float mlo, mhi; };
 
   // the first of four consecutive values of half h (values 0..3 or 4..7) of chunk (q, m); the
-  // chunk takes them in the order 0, 2, 1, 3
+  // chunk takes them in the order 0, 2, 1, 3 (SWAP)
   __device__ static int xoff4(int q, int m, int h) { return 64 * q + 32 * h + 4 * m; }
-  static constexpr bool SWAP = true;
 
   __device__ static void load(const uint8_t *blk, int q, Raw &r) {
     r.h = ldw16(blk);
@@ -61,42 +61,6 @@ struct WQ4K {
     const uint4 h = r.h;
     const int k = 16 * (q & 1);
     // get_scale_min_k4 (src/Quants.cs:321-330) for sub-blocks 2q, 2q + 1
-    const uint32_t S = q < 2 ? (h.y & 0x3F3F3F3Fu) : ((h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u));
-    const uint32_t M = q < 2 ? (h.z & 0x3F3F3F3Fu) : (((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u));
-    const float sclo = (float)((S >> k) & 0xFF), schi = (float)((S >> (k + 8)) & 0xFF);
-    const _Float16 a = (_Float16)sclo, b = (_Float16)(schi * 0.0625f);
-    const _Float16 na = (_Float16)(-1024.f * sclo), nb = (_Float16)(-64.f * schi);
-    return Scale{fh2{a, a}, fh2{na, na}, fh2{b, b}, fh2{nb, nb}, (float)((M >> k) & 0xFF),
-                 (float)((M >> (k + 8)) & 0xFF)};
-  }
-
-  __device__ static void frag(const Raw &r, const Scale &s, int, int m, fh8 (&f)[1]) {
-    const uint32_t qd[8] = {r.q0.x, r.q0.y, r.q0.z, r.q0.w, r.q1.x, r.q1.y, r.q1.z, r.q1.w};
-    const uint32_t D = qd[m], D8 = D >> 8;
-    const fh2 p0 = __builtin_elementwise_fma(as_fh2((D & 0x000F000Fu) | 0x64006400u), s.sl, s.nl);
-    const fh2 p1 = __builtin_elementwise_fma(as_fh2((D8 & 0x000F000Fu) | 0x64006400u), s.sl, s.nl);
-    const fh2 p2 = __builtin_elementwise_fma(as_fh2((D & 0x00F000F0u) | 0x64006400u), s.sh, s.nh);
-    const fh2 p3 = __builtin_elementwise_fma(as_fh2((D8 & 0x00F000F0u) | 0x64006400u), s.sh, s.nh);
-    f[0] = fh8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-  }
-  __device__ static float d(const Raw &r) { return half_lo(r.h.x); }
-  __device__ static float dmin(const Raw &r) { return half_hi(r.h.x); }
-};
-
-// Q4_K centred: (n - 8) sc, exact (at most 8 * 63), and per sub-block the factor 8 d sc - dmin m of its
-// sum of x, rounded once (both products are exact in fp32).
-struct WQ4KC {
-  static constexpr int BYTES = 144, NF = 1;
-  static constexpr bool MINS = true, SWAP = true;
-  typedef WQ4K::Raw Raw;
-  struct Scale { fh2 sl, sh; float mlo, mhi; };
-
-  __device__ static int xoff4(int q, int m, int h) { return WQ4K::xoff4(q, m, h); }
-  __device__ static void load(const uint8_t *blk, int q, Raw &r) { WQ4K::load(blk, q, r); }
-
-  __device__ static Scale scale(const Raw &r, int q) {
-    const uint4 h = r.h;
-    const int k = 16 * (q & 1);
     const uint32_t S = q < 2 ? (h.y & 0x3F3F3F3Fu) : ((h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u));
     const uint32_t M = q < 2 ? (h.z & 0x3F3F3F3Fu) : (((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u));
     const float sclo = (float)((S >> k) & 0xFF), schi = (float)((S >> (k + 8)) & 0xFF);

@@ -9,13 +9,15 @@
 //
 // Arithmetic, at fp32's precision: a weight is an exact fp16 integer (wl_fmma_codec.h), a
 // token's 256 activations of a super-block are scaled by a power of two and split into
-// hi = fp16(x f), lo = fp16(x f - hi), 22 significant bits, and the exact products accumulate into
-// fp32, the parts apart (the lo sums round 2^11 times finer). Q4_K's quants enter as n - 8, with the
-// sub-block's 8 d sc - dmin m as the factor of its sum of x (a 16x16x4 fp32 MFMA): the two large
-// terms that nearly cancel in n sc and the minimum never become sums of their own (error against 64
-// bits at 300 tokens of 128 experts 5.2e-7 with n, 3.7e-7 row by row in fp32). A super-block's sum is
-// then scaled by d and 1/f and added in order, so a token's result depends neither on the other tokens
-// nor on its place in a tile.
+// hi = fp16(x f), lo = fp16(x f - hi), 22 significant bits down to 2^-17 of the 256's largest value
+// (2^-39 of it below), and the exact products accumulate into fp32, the parts apart (the lo sums round
+// 2^11 times finer). Q4_K's quants enter as n - 8, with the sub-block's 8 d sc - dmin m as the factor of
+// its sum of x (a 16x16x4 fp32 MFMA): the two large terms that nearly cancel in n sc and the minimum
+// never become sums of their own (error against 64 bits at 300 tokens of 128 experts 5.2e-7 with n, 2.4e-7
+// so, 3.7e-7 row by row in fp32; over 24 drawn shapes, some with columns 30 to 10,000 times the others,
+// 2.2e-7 to 2.8e-7 against 2.9e-7 to 4.2e-7 row by row). A super-block's sum is then scaled by d and 1/f
+// and added in order, so a token's result depends neither on the other tokens nor on its place in a
+// tile.
 //
 // Launches: route (one wave per token), plan (one workgroup per expert numbers its pairs), the
 // tokens' parts, gate/up with the SiLU, the hidden rows' parts, down, combine.
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(256) void moe_parts_kernel(const float *__restrict_
   fh8 o;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    // the chunk's order of each four values (WQ4KC: 0, 2, 1, 3)
+    // the chunk's order of each four values (WQ4K: 0, 2, 1, 3)
     const int j = C::SWAP && (i & 3) == 1 ? i + 1 : C::SWAP && (i & 3) == 2 ? i - 1 : i;
     const float X = v[j] * f;
     const _Float16 hi = (_Float16)X;
@@ -385,7 +387,7 @@ static hipError_t parts_launch(int type, const float *x, int64_t rows, int cols,
   const int nsb = cols / 256;
   const dim3 grid((unsigned)((rows * nsb + 3) / 4));
   if (type == 12)
-    hipLaunchKernelGGL(moe_parts_kernel<WQ4KC>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
+    hipLaunchKernelGGL(moe_parts_kernel<WQ4K>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
   else
     hipLaunchKernelGGL(moe_parts_kernel<WQ6K>, grid, dim3(256), 0, st, x, rows, nsb, (uint4 *)p, (float *)sums, (float *)inv);
   return hipGetLastError();
@@ -436,7 +438,7 @@ hipError_t moe_many_launch(const MoeLaunch &l, void *scratch, hipStream_t st) {
   g.inv = (const float *)(b + s.xinv);
   g.by_pair = 0;
   g.y = (float *)(b + s.h);
-  e = l.gu_type == 12 ? many_gemm<WQ4KC, true>(g, nt, max_tiles, st) : many_gemm<WQ6K, true>(g, nt, max_tiles, st);
+  e = l.gu_type == 12 ? many_gemm<WQ4K, true>(g, nt, max_tiles, st) : many_gemm<WQ6K, true>(g, nt, max_tiles, st);
   if (e != hipSuccess) return e;
   if ((e = parts_launch(l.d_type, g.y, P, l.ff, b + s.hp, b + s.hsum, b + s.hinv, st)) != hipSuccess) return e;
   MoeGemm d = g;
@@ -451,7 +453,7 @@ hipError_t moe_many_launch(const MoeLaunch &l, void *scratch, hipStream_t st) {
   d.inv = (const float *)(b + s.hinv);
   d.by_pair = 1;
   d.y = (float *)(b + s.y);
-  e = l.d_type == 12 ? many_gemm<WQ4KC, false>(d, nt, max_tiles, st) : many_gemm<WQ6K, false>(d, nt, max_tiles, st);
+  e = l.d_type == 12 ? many_gemm<WQ4K, false>(d, nt, max_tiles, st) : many_gemm<WQ6K, false>(d, nt, max_tiles, st);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(moe_many_combine_kernel, dim3((unsigned)(((int64_t)l.T * l.embd / 4 + 255) / 256)), dim3(256), 0, st,
                      m, d.y, l.T, l.k, l.embd, l.out);
