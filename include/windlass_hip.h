@@ -195,8 +195,9 @@ int wl_set_int_dot(wl_ctx *ctx, int on);
 /* The float arithmetic of ForwardBatch (src/Transformer.cs:127-170; MatMulEach, :544-561) on the
  * matrix cores, for an engine started with --batch N (EngineOptions.Batch, src/Engine.cs:21,65;
  * src/Program.cs:213). Off by default. When on, every float decode GEMV of Q4_K and Q6_K weights
- * (wl_matmul(_dev), the fused q/k/v and SwiGLU entries, the layer entries; 1-8 tokens per pass)
- * runs on fp16 MFMA with each token's x split exactly into two fp16 parts: results within the
+ * (wl_matmul(_dev), the fused q/k/v and SwiGLU entries, the layer entries; 1-8 tokens per pass, 1-16
+ * in wl_gate_up_dev and wl_layer_batch_dev) runs on fp16 MFMA with each token's x as two fp16 parts
+ * (22 significant bits down to 2^-17 of the largest of 2048 values): results within the
  * float bar of the reference's DotRow, and a token's bits are the same whatever the number of
  * tokens in the call, so a batched sequence gets the bits it gets alone in the same mode. The
  * bits differ from the default (VALU) arithmetic's in the last places; switch it per context
@@ -223,8 +224,8 @@ int wl_matmul_dev(wl_ctx *ctx, const wl_weight *w, int32_t expert, const float *
 
 /* MatMul followed by Layer's residual add (src/Transformer.cs:224,231): d_y [T][rows] +=
  * (W x) * rs, the product rounded to float first and the add as two roundings, so the bits
- * equal wl_matmul_dev then wl_residual_dev. Up to 8 tokens the add is the GEMV's own store (no
- * extra launch). */
+ * equal wl_matmul_dev then wl_residual_dev. Up to 8 tokens, and for prompts over Q8_0, Q4_K, Q5_K,
+ * Q6_K and IQ4_XS rows, the add is the product's own store (no extra launch). */
 int wl_matmul_add_dev(wl_ctx *ctx, const wl_weight *w, int32_t expert, const float *d_x, int32_t T,
                       float *d_y, float rs);
 
@@ -245,7 +246,8 @@ int wl_dequant_dev(wl_ctx *ctx, const wl_weight *w, int64_t row0, int64_t nrows,
  * on = 1 (the default) routes, plans, runs gate/up and down and combines in one launch where
  * the shapes allow it (Q4_K/Q6_K experts, hidden and FFN up to 2048, up to 64 token-expert
  * pairs per pass, up to 256 experts, float products); on = 0 always runs the launch chain
- * (route+plan, gate/up, down, combine). Both give the same bits. */
+ * (route+plan, gate/up, down, combine). Both give the same bits. Prompts on the matrix cores
+ * (wl_moe_ffn_dev) are not concerned. */
 int wl_set_moe_one_launch(wl_ctx *ctx, int on);
 
 /* Fault injection for the one-launch MoE's error path (no counterpart in the reference): the
@@ -256,7 +258,10 @@ int wl_set_moe_one_launch(wl_ctx *ctx, int on);
 int wl_debug_moe_patience(wl_ctx *ctx, int32_t polls);
 
 /* wl_moe_ffn on device buffers (logits, x, out in HBM). Asynchronous: a one-launch failure is
- * reported by the next wl_sync. */
+ * reported by the next wl_sync. More than 8 tokens of Q4_K / Q6_K experts whose rows are whole blocks
+ * of 256 (float products) run on fp16 MFMA with x and the hidden rows as two fp16 parts, each expert's
+ * weights read once; a token's bits do not depend on the others there, and differ in the last places
+ * from passes of up to 8 (which wl_moe_ffn and wl_layer_batch_dev always take). */
 int wl_moe_ffn_dev(wl_ctx *ctx, const float *d_logits, int32_t k, int32_t renorm,
                    const wl_weight *gate_exps, const wl_weight *up_exps,
                    const wl_weight *down_exps, const float *d_x, int32_t T, float *d_out);
@@ -285,7 +290,10 @@ int wl_kv_store_dev(wl_ctx *ctx, const float *d_k, const float *d_v, int32_t T, 
                     uint16_t *d_V, int32_t pos0);
 
 /* Attention (src/Transformer.cs:351-393): row t attends to positions 0..pos0+t of the fp16
- * caches; softmax with exp and the denominator in double; grouped KV heads. */
+ * caches; grouped KV heads. Softmax with exp and the denominator in double up to 15 rows and for
+ * other head dims than 64 and 128; 16 rows and more of those run on fp16 MFMA with the queries and
+ * probabilities as two fp16 parts, exp2 in fp32 and the denominator in fp32 per 64 positions, in
+ * double across them, within the same bar and no further from the exact result. */
 int wl_attention_dev(wl_ctx *ctx, const float *d_q, int32_t T, int32_t heads, int32_t kv_heads, int32_t head_dim,
                      const uint16_t *d_K, const uint16_t *d_V, int32_t pos0, float scale, float *d_out);
 
@@ -344,7 +352,7 @@ int wl_scale_dev(wl_ctx *ctx, float *d_x, int64_t n, float s);
  * rows pos0.. of the fp16 caches d_K / d_V [positions][kv_heads * head_dim]. Every activation
  * stays in HBM (the context's scratch); stream-ordered, no host wait. Up to 8 tokens the
  * products are the decode GEMVs (o and down add into x in their own store); more tokens take
- * the GEMMs. The caches must hold pos0 + T positions: the library cannot check their size.
+ * the GEMMs (and MoE prompts wl_moe_ffn_dev's). The caches must hold pos0 + T positions: the library cannot check their size.
  * Like the reference's RopeTable (src/Transformer.cs:396-414) the context keeps the RoPE angles
  * of the positions it has seen, for the last setting (rope dims, base, frequency scale,
  * rope_freqs pointer); each entry records the frequency factors it was made with, and an entry
@@ -356,7 +364,7 @@ int wl_layer_dev(wl_ctx *ctx, const wl_layer_desc *layer, float *d_x, int32_t T,
  * of its own sequence, at position pos[i] of cache slot slot[i] (host arrays, checked: slots
  * distinct and below `slots`, positions below slot_positions). d_K / d_V are this layer's pools
  * [slots][slot_positions][kv_heads * head_dim]. Every product runs the GEMV in passes of at most
- * 8 rows (EachToken), so row i's bits equal wl_layer_dev of that token alone on its sequence. */
+ * 8 rows (EachToken; 16 where wl_set_float_mma's kernels take them), so row i's bits equal wl_layer_dev of that token alone on its sequence. */
 int wl_layer_batch_dev(wl_ctx *ctx, const wl_layer_desc *layer, float *d_x, int32_t N, const int32_t *pos,
                        const int32_t *slot, int32_t slots, int32_t slot_positions, uint16_t *d_K, uint16_t *d_V);
 

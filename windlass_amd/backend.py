@@ -147,7 +147,7 @@ class Context:
     @property
     def FloatMma(self):
         """ForwardBatch's float products (src/Transformer.cs:127-170) on the matrix cores: Q4_K
-        and Q6_K decode GEMVs of 1-8 tokens on fp16 MFMA with x split exactly into two fp16
+        and Q6_K decode GEMVs of 1-16 tokens on fp16 MFMA with x split into two fp16
         parts, a token's bits independent of the batch. Off by default."""
         return getattr(self, "_float_mma", False)
 

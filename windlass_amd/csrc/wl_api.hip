@@ -65,7 +65,7 @@ struct wl_ctx {
   hipStream_t stream;
   hipStream_t copy;  // stage uploads (default priority), created on first use
   int int_dot;  // Transformer.IntDot (src/Transformer.cs:23)
-  int float_mma;  // wl_set_float_mma: Q4_K / Q6_K decode GEMVs of 1-8 tokens on the matrix cores
+  int float_mma;  // wl_set_float_mma: Q4_K / Q6_K decode GEMVs on the matrix cores
   int moe_chain;  // wl_set_moe_one_launch(0): the MoE entries always run the launch chain
   bool capturing = false;  // between wl_capture_begin and wl_capture_end
   unsigned moe_launches;  // one-launch MoE launches so far (their counter sets alternate)
@@ -1339,7 +1339,7 @@ extern "C" int wl_embed_dev_ids(wl_ctx *c, const wl_weight *embd, const int32_t 
 
 // Transformer.Layer (src/Transformer.cs:177-232) with every activation in HBM. rm/max_n: the
 // rows' positions and cache slots (a batch step) and the most positions a row attends to;
-// each: every product in GEMV passes of at most 8 rows, so a row's bits do not depend on the
+// each: every product in GEMV passes of at most 8 rows (16 on the matrix cores), so a row's bits do not depend on the
 // batch (ForwardBatch's EachToken, src/Transformer.cs:127-170).
 // The rows' RoPE angles in the context's table: positions hpos[0..T-1] (host values), or pos0 ..
 // pos0 + T - 1 when hpos is null. Missing positions are filled by one launch over their range,

@@ -12,7 +12,7 @@
 // Arithmetic, at fp32's precision (Attention, src/Transformer.cs:351-393): the caches' fp16 keys
 // and values are exact operands. A query row is scaled by a power of two and split into
 // hi = fp16(q f), lo = fp16(q f - hi): 22 significant bits down to 2^-17 of the head's largest value,
-// 2^-40 of that value below; exact products, fp32 sums. The probabilities are exp2 in fp32 of
+// 2^-39 of that value below; exact products, fp32 sums. The probabilities are exp2 in fp32 of
 // (score - running maximum) times the scale: the difference first, so that the argument's rounding
 // is relative to the argument (a maximum scaled and rounded by itself, 14 up, left 1.6e-7 in flat
 // softmaxes, and past scores of 2^26 no probability near 1). They enter the products as two fp16

@@ -280,7 +280,8 @@ struct FQ6K {
 
 // ------------------------------------------------------------------------------------ kernel
 // Loads in flight per wave: PF work items (one matrix's super-block) ahead of the one computed,
-// as many as the register budget (128 VGPRs, four waves per SIMD) holds without spilling.
+// as many as the register budget (128 VGPRs, four waves per SIMD) holds. Kernels of one token set do not
+// spill; of two sets, q/k/v of both formats spill 8 registers, one Q6_K matrix 4 and a Q6_K pair 32.
 #ifndef WL_FMMA_PF_Q4K
 #define WL_FMMA_PF_Q4K 1
 #endif

@@ -1,4 +1,4 @@
-// wl_gemm_short.h - prompts of 9 to a few hundred tokens over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS
+// wl_gemm_short.h - prompts of 9 to 128 tokens over Q8_0, Q4_K, Q5_K, Q6_K and IQ4_XS
 // rows on the bf16 matrix cores (the batch branch of Transformer.MatMul,
 // src/Transformer.cs:526-536): host interface.
 #pragma once

@@ -1,9 +1,10 @@
-// wl_gemm_short.hip - prompts of 9 to a few hundred tokens on the bf16 matrix cores.
+// wl_gemm_short.hip - prompts of 9 to 128 tokens on the bf16 matrix cores.
 //
 // What bounds it: the weights' bytes (an 8B layer's 132 MB are 20 us at 6.5 TB/s) and the decode
 // (about 3 VALU instructions a weight, 19 us for the layer), not the products. So every weight is
-// read and decoded once per 128 tokens, straight from memory into the registers of the lane whose
-// matrix operand it is: no LDS for weights, no padding of the tokens past the next 16.
+// read and decoded once for all tokens, straight from memory into the registers of the lane whose
+// matrix operand it is: no LDS for weights. Tokens are multiplied in tiles of 16, 5 and 7 tiles as 6
+// and 8 (the last one again). The kernels of 8 tiles by 32 rows on eight waves spill 12 to 15 registers.
 //
 // A workgroup owns 16 R rows and splits K over its KW waves, whose sums meet in LDS at the end in
 // wave order: the launch fills the device without partial planes in memory and a launch to add
@@ -345,7 +346,7 @@ __device__ __forceinline__ void short_body(const ShortArgs &a, const ShortMat &m
           g += red[((w * TR + t) * 2) * 256 + e];
           u += red[((w * TR + t) * 2 + 1) * 256 + e];
         }
-        if (t1 + t < NT && tok < a.tiles * 16) {  // tokens past T in the last tile: copies of token T - 1
+        if (t1 + t < NT && tok < a.tiles * 16) {  // tokens past T in the last tile: any value, never stored in y
           const int row = row0 + (e & 15);
           const __bf16 h = (__bf16)silu_mul(g, u);
           a.hf[frag_at(tok, row & ~7, mat.rows, a.hord) * 8 + (row & 7)] = __builtin_bit_cast(uint16_t, h);
@@ -388,7 +389,9 @@ __global__ __launch_bounds__(64 * KW) void short_kernel(ShortArgs a) {
 }
 
 // ------------------------------------------------------------------------------- operands
-// A thread per 16-byte piece; tokens past T in the last tile repeat token T - 1 (never stored).
+// A thread per 16-byte piece; tokens past T in the last tile repeat token T - 1 here. Pieces that a norm
+// or gate and up write leave those places as they are or hold any value: an MFMA's columns are
+// independent, and the results of tokens past T are never stored.
 __global__ __launch_bounds__(256) void short_frag_kernel(const float *__restrict__ x, int T, int cols, int64_t n,
                                                          int ord, uint4 *__restrict__ xf) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;

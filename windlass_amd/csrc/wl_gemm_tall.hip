@@ -289,7 +289,8 @@ struct TIQ4XS {
 // xf fragment (j, s), j = token block of 32, s = step of 32 columns, is 2 x 64 lanes x 16 bytes at
 // xf + (j * nsteps + s) * 128: half u (columns 16u .. 16u+15 of the step), lane l holds token
 // 32j + l%32, columns 32s + 16u + 8(l/32) .. +7 as bf16 (round to nearest even). Tokens past T
-// repeat token T - 1 (their results are never stored).
+// repeat token T - 1, or where a norm wrote the fragments hold any value (their results are never
+// stored, and an MFMA's columns are independent).
 // One workgroup per (token block j, 8 steps): the 32 tokens' 256 columns come in as 1 KB rows
 // (a wave reads one row's 256 floats), go through LDS as bf16, and leave as the 8 fragments
 // (j, s0 .. s0+7), 16 KB contiguous in xf.
