@@ -228,7 +228,8 @@ def test_fmma_leaves_other_formats_alone(ctx):
 
 @pytest.mark.parametrize("t", TYPES, ids=lambda t: t.name)
 @pytest.mark.parametrize("T", [9, 13, 16, 21])  # one pass of two token sets, and a pass more
-@pytest.mark.parametrize("rows,cols", [(37, 2304), (4128, 512)])  # fewer tiles than CUs, and more than a round's waves
+# fewer tiles than CUs, more than a round's waves, and more 2048-column units than CUs
+@pytest.mark.parametrize("rows,cols", [(37, 2304), (4128, 512), (20, 520 * 2048)])
 def test_fmma_wide_pass_rows_equal_single_token_bitwise(ctx, t, T, rows, cols):
     g, u = (ctx.upload(t, blocks(t, rows, cols, seed=40 + i), rows, cols) for i in range(2))
     x = _dev(np.random.default_rng(T).standard_normal((T, cols), dtype=np.float32))

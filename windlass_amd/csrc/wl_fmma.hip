@@ -444,23 +444,39 @@ hipError_t fmma_run(const GemvMat *mats, int nmat, int nm, const float *x, int l
   a.x = x;
   a.ldx = ldx;
   a.T = T;
-  // One round of 16 resident waves per CU (two workgroups, or one of 16 waves), the workgroups shared
-  // out by the matrices' tiles: tiles of few rows go to all CUs, a few waves of each (grouped eight to
-  // a workgroup, 8B q/k/v at 8 tokens used 96 workgroups of 512 and took 18.8 us).
+  // Workgroups per unit: as many as give every wave a tile, but at least one a CU (tiles of few rows
+  // go to all CUs, a few waves of each) and at most the 16 resident waves of each (two workgroups, or one
+  // of 16 waves): every workgroup prepares the tokens' parts anew, and one past the resident ones runs
+  // in a round of its own. At 8 tokens, 8B q/k/v 18.8 us on 96 workgroups of full waves, 70B q/k/v 33.0 on
+  // 516 and 27.0 on 320, o 16.8 on 512 and 14.3 on 256. Shared out by the matrices' tiles.
   const int W = fm_waves(T > 8 ? 2 : 1);
   int64_t tiles = 0;
   for (int i = 0; i < nmat; i++) tiles += (mats[i].rows + 15) / 16;
-  int64_t want = (int64_t)num_cu * 16 / W / a.u;
-  if (want < 1) want = 1;
+  int64_t want = (tiles + W - 1) / W;
+  if (want < num_cu / a.u) want = num_cu / a.u;
+  if (want > (int64_t)num_cu * 16 / W / a.u) want = (int64_t)num_cu * 16 / W / a.u;
+  int64_t share[GEMV_MAX_MATS], left = want;
+  for (int i = 0; i < nmat; i++) {
+    const int64_t t = (mats[i].rows + 15) / 16, n = want * t / tiles;
+    share[i] = n < 1 ? 1 : n > t ? t : n;
+    left -= share[i];
+  }
+  for (; left > 0; left--) {  // what the shares' rounding left: to the matrix with the most tiles a workgroup
+    int best = -1;
+    for (int i = 0; i < nmat; i++) {
+      const int64_t t = (mats[i].rows + 15) / 16;
+      if (share[i] < t && (best < 0 || t * share[best] > (int64_t)((mats[best].rows + 15) / 16) * share[i])) best = i;
+    }
+    if (best < 0) break;
+    share[best]++;
+  }
   float *part = scratch;
   int gx = 0;
   for (int i = 0; i < nmat; i++) {
     const GemvMat &m = mats[i];
     a.m[i] = BatchMat{m.w, m.w2, m.row_bytes, part, m.y, m.ldy, m.rows, m.type, gx, m.add, m.rs};
     part += (int64_t)a.u * nm * T * m.rows;
-    const int64_t t = (m.rows + 15) / 16;
-    int64_t n = (want * t + tiles - 1) / tiles;
-    gx += (int)(n > t ? t : n);
+    gx += (int)share[i];
   }
   int kinds = 0;
   for (int i = 0; i < nmat; i++) kinds |= mats[i].type == 12 ? 1 : 2;
