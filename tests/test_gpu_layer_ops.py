@@ -105,6 +105,23 @@ def test_rope(ctx, neox, heads, hd, n, base, fs, factors, positions):
         assert np.array_equal(r, x.reshape(T, heads, hd)[:, :, n:])
 
 
+# either side of the rows that take their angles once a row, of each split of a row over workgroups, and
+# more than 256 pairs of a head
+@pytest.mark.parametrize("T", [64, 65, 127, 128, 511, 512])
+@pytest.mark.parametrize("heads,hd,n,neox,at", [(5, 64, 48, 0, False), (3, 128, 128, 1, True), (2, 640, 600, 0, False)])
+def test_rope_rows_equal_single_rows_bitwise(ctx, heads, hd, n, neox, at, T):
+    rng = np.random.default_rng(T + hd)
+    pos = rng.integers(0, 9000, T).astype(np.int32)
+    x, freqs = rng.standard_normal((T, heads * hd), dtype=F32), (1 + rng.random(n // 2)).astype(F32)
+    many, one, dpos, df = dev(x), dev(x), dev(pos), dev(freqs)
+    rope = lambda y, rows, p0, dp: check(load().wl_rope_dev(  # noqa: E731
+        ctx.handle, y, rows, heads, hd, n, neox, p0, dp, 10000.0, 1.0, P(df)))
+    rope(P(many), T, 7, P(dpos) if at else None)
+    for t in range(T):
+        rope(P(one[t:t + 1]), 1, 7 + t, P(dpos[t:t + 1]) if at else None)
+    assert np.array_equal(host(ctx, many).view(np.uint32), host(ctx, one).view(np.uint32))
+
+
 def test_kv_store_rounds_to_nearest_even(ctx):
     rng = np.random.default_rng(3)
     kd, T, pos0, cap = 96, 5, 11, 20

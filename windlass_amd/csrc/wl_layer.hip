@@ -200,53 +200,85 @@ __global__ __launch_bounds__(64) void rope_table_kernel(float4 *__restrict__ tab
 
 // RoPE on q (H heads) and k (KH heads) of row t, and ToHalf of the row's keys and values into
 // cache row pos0 + t, or row pos[t] of slot slot[t] (slots of cap positions) for a batch step
-// (src/Transformer.cs:204-215,342-348). A workgroup takes the angles of 256 pairs of its row once, into
-// LDS (a thread per pair; a thread per pair and head took the double cosine and sine H + KH times:
-// 2,048 rows of 40 heads 90 us), then a thread per rotated pair of the q and k heads and per key/value
-// column (the value's store, and the key's for columns past rope_dims), both shared by the gridDim.y
-// workgroups of a row. k, v and the caches are null for RoPE on one tensor.
-__global__ __launch_bounds__(256) void rope_qkv_kernel(float *__restrict__ q, int64_t ldq, int H, float *__restrict__ k,
-                                                       const float *__restrict__ v, int KH, int hd, int n, int neox,
-                                                       const int *__restrict__ pos, int pos0, double theta_scale,
-                                                       double freq_scale, const float *__restrict__ freqs,
-                                                       uint16_t *__restrict__ Kc, uint16_t *__restrict__ Vc,
-                                                       const int *__restrict__ slot, int64_t cap) {
+// (src/Transformer.cs:204-215,342-348): a work item per rotated pair of every q and k head, and one per
+// key/value column (the value's store, and the key's for columns past rope_dims). k, v and the
+// caches are null for RoPE on one tensor.
+struct RopeRow {
+  float *q;
+  int64_t ldq;
+  int H;
+  float *k;
+  const float *v;
+  int KH, hd, n, neox, pos0;
+  const int *pos;
+  double theta_scale, freq_scale;
+  const float *freqs;
+  uint16_t *Kc, *Vc;
+  const int *slot;
+  int64_t cap;
+
+  __device__ int position(int t) const { return pos ? pos[t] : pos0 + t; }
+  __device__ int64_t cache_row(int t) const {
+    return (slot ? (int64_t)slot[t] * cap + position(t) : (int64_t)(pos0 + t)) * KH * hd;
+  }
+  // pair i of head `head` (q's, then k's) by the angle (c, s)
+  __device__ void rotate(int t, int64_t crow, int head, int i, float c, float s) const {
+    float y0, y1;
+    int a, b;
+    if (head < H) {
+      rope_pair(q + (int64_t)t * ldq + (int64_t)head * hd, i, n, neox, c, s, y0, y1, a, b);
+    } else {
+      const int kh = head - H;
+      rope_pair(k + (int64_t)t * KH * hd + (int64_t)kh * hd, i, n, neox, c, s, y0, y1, a, b);
+      if (Kc) {
+        Kc[crow + kh * hd + a] = to_half(y0);
+        Kc[crow + kh * hd + b] = to_half(y1);
+      }
+    }
+  }
+  __device__ void column(int t, int64_t crow, int j) const {
+    Vc[crow + j] = to_half(v[(int64_t)t * KH * hd + j]);
+    if (j % hd >= n) Kc[crow + j] = to_half(k[(int64_t)t * KH * hd + j]);
+  }
+};
+
+// Up to kRopeItemRows rows: a thread per work item, each pair's angle taken by its own thread. The launch
+// is as long as one angle's chain of products (70B layer, 8 rows 5.0 us; with the angles through LDS and
+// a barrier 7.2, and 6.2 with as many workgroups as here).
+__global__ __launch_bounds__(256) void rope_items_kernel(RopeRow R) {
+  const int t = blockIdx.y, half = R.n / 2, it = blockIdx.x * 256 + threadIdx.x, npairs = (R.H + R.KH) * half;
+  const int64_t crow = R.cache_row(t);
+  float c = 0.f, s = 0.f;  // every lane runs the angle product (uniform trip count)
+  if (half > 0) rope_cs(R.position(t), it < npairs ? it % half : 0, half, R.theta_scale, R.freq_scale, R.freqs, c, s);
+  if (it < npairs) R.rotate(t, crow, it / half, it % half, c, s);
+  else if (it < npairs + R.KH * R.hd && R.Vc) R.column(t, crow, it - npairs);
+}
+
+// More rows: a workgroup takes the angles of 256 pairs of its row once, into LDS (a thread per pair; a
+// thread per pair and head took the double cosine and sine H + KH times: 2,048 rows of 40 heads 90 us
+// against 31), then a thread per work item, shared by the gridDim.y workgroups of a row.
+__global__ __launch_bounds__(256) void rope_qkv_kernel(RopeRow R) {
   __shared__ float2 angle[256];  // (cos, sin)
-  const int t = blockIdx.x, half = n / 2, KD = KH * hd, tid = threadIdx.x;
+  const int t = blockIdx.x, half = R.n / 2, KD = R.KH * R.hd, heads = R.H + R.KH, tid = threadIdx.x;
   const int first = blockIdx.y * 256 + tid, step = gridDim.y * 256;
-  const int p = pos ? pos[t] : pos0 + t;
-  const int64_t crow = (slot ? (int64_t)slot[t] * cap + p : (int64_t)(pos0 + t)) * KD;
+  const int p = R.position(t);
+  const int64_t crow = R.cache_row(t);
   for (int i0 = 0; i0 < half; i0 += 256) {
     const int cn = min(256, half - i0);
     if (i0) __syncthreads();  // the pairs before are rotated
     if ((tid & ~63) < cn) {   // whole waves run the angle product (uniform trip count)
       float c, s;
-      rope_cs(p, tid < cn ? i0 + tid : 0, half, theta_scale, freq_scale, freqs, c, s);
+      rope_cs(p, tid < cn ? i0 + tid : 0, half, R.theta_scale, R.freq_scale, R.freqs, c, s);
       if (tid < cn) angle[tid] = make_float2(c, s);
     }
     __syncthreads();
-    for (int it = first; it < (H + KH) * cn; it += step) {
-      const int head = it / cn, i = i0 + it % cn;
+    for (int it = first; it < heads * cn; it += step) {
       const float2 cs = angle[it % cn];
-      float y0, y1;
-      int a, b;
-      if (head < H) {
-        rope_pair(q + (int64_t)t * ldq + (int64_t)head * hd, i, n, neox, cs.x, cs.y, y0, y1, a, b);
-      } else {
-        const int kh = head - H;
-        rope_pair(k + (int64_t)t * KD + (int64_t)kh * hd, i, n, neox, cs.x, cs.y, y0, y1, a, b);
-        if (Kc) {
-          Kc[crow + kh * hd + a] = to_half(y0);
-          Kc[crow + kh * hd + b] = to_half(y1);
-        }
-      }
+      R.rotate(t, crow, it / cn, i0 + it % cn, cs.x, cs.y);
     }
   }
-  if (Vc)
-    for (int j = first; j < KD; j += step) {
-      Vc[crow + j] = to_half(v[(int64_t)t * KD + j]);
-      if (j % hd >= n) Kc[crow + j] = to_half(k[(int64_t)t * KD + j]);
-    }
+  if (R.Vc)
+    for (int j = first; j < KD; j += step) R.column(t, crow, j);
 }
 
 // ToHalf (src/Transformer.cs:342-348) of one token's keys and values.
@@ -948,25 +980,33 @@ hipError_t rms_norm_frag_launch(const float *x, int rows, int64_t dim, const flo
   return hipGetLastError();
 }
 
-// Workgroups of a row: few rows spread over the CUs, many take their angles once.
-static unsigned rope_split(int T) { return T >= 512 ? 1 : T >= 128 ? 2 : 8; }
+// Where every row's angles once through LDS begin to win: 64 rows (8B layer 6.2 us either way; 45 rows
+// 5.4 with a thread per item and 6.2, 100 rows 7.9 and 6.5; 70B 7.0 and 7.8, 10.5 and 8.6).
+constexpr int kRopeItemRows = 64;
+
+static hipError_t rope_rows(const RopeRow &R, int T, hipStream_t st) {
+  if (T <= 0) return hipSuccess;
+  if (T <= kRopeItemRows) {
+    const int64_t items = (int64_t)(R.H + R.KH) * (R.n / 2) + (R.Vc ? (int64_t)R.KH * R.hd : 0);
+    if (items > 0) hipLaunchKernelGGL(rope_items_kernel, dim3(blocks_of(items, 256), T), dim3(256), 0, st, R);
+  } else {
+    // few rows spread over the CUs, many take their angles once
+    hipLaunchKernelGGL(rope_qkv_kernel, dim3((unsigned)T, T >= 512 ? 1 : T >= 128 ? 2 : 8), dim3(256), 0, st, R);
+  }
+  return hipGetLastError();
+}
 
 hipError_t rope_launch(float *x, int64_t ldx, int T, int heads, int hd, int n, int neox, const int *pos, int pos0,
                        double base, double freq_scale, const float *freqs, hipStream_t st) {
-  if (T <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rope_qkv_kernel, dim3((unsigned)T, rope_split(T)), dim3(256), 0, st, x, ldx, heads, nullptr,
-                     nullptr, 0, hd, n, neox, pos, pos0, pow(base, -2.0 / n), freq_scale, freqs, nullptr, nullptr,
-                     nullptr, (int64_t)0);
-  return hipGetLastError();
+  return rope_rows(RopeRow{x, ldx, heads, nullptr, nullptr, 0, hd, n, neox, pos0, pos, pow(base, -2.0 / n), freq_scale,
+                           freqs, nullptr, nullptr, nullptr, 0}, T, st);
 }
 
 hipError_t rope_kv_launch(float *q, float *k, const float *v, int T, int H, int KH, int hd, int n, int neox,
                           int pos0, double base, double freq_scale, const float *freqs, uint16_t *Kc, uint16_t *Vc,
                           const RowMap &rm, hipStream_t st) {
-  if (T <= 0) return hipSuccess;
-  hipLaunchKernelGGL(rope_qkv_kernel, dim3((unsigned)T, rope_split(T)), dim3(256), 0, st, q, (int64_t)H * hd, H, k, v,
-                     KH, hd, n, neox, rm.pos, pos0, pow(base, -2.0 / n), freq_scale, freqs, Kc, Vc, rm.slot, rm.cap);
-  return hipGetLastError();
+  return rope_rows(RopeRow{q, (int64_t)H * hd, H, k, v, KH, hd, n, neox, pos0, rm.pos, pow(base, -2.0 / n), freq_scale,
+                           freqs, Kc, Vc, rm.slot, rm.cap}, T, st);
 }
 
 hipError_t kv_store_launch(const float *k, const float *v, int64_t n, uint16_t *K, uint16_t *V, hipStream_t st) {
