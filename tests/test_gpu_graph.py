@@ -100,3 +100,68 @@ def test_capture_refuses_scratch_growth():
         assert all(np.isfinite(v).all() for v in got.values())
     finally:
         ctx.close()
+
+
+class Prompt:
+    """An attention layer's prompt of T tokens after 30 and a prompt through 16 experts, in one run."""
+    SHAPES = {"attn_q": (Q4_K, 512, 512), "attn_k": (Q4_K, 128, 512), "attn_v": (Q6_K, 128, 512),
+              "attn_output": (Q4_K, 512, 512), "ffn_gate": (Q4_K, 1024, 512), "ffn_up": (Q4_K, 1024, 512),
+              "ffn_down": (Q6_K, 512, 1024)}
+
+    def __init__(self, ctx, T, seed):
+        from windlass_amd import LayerDesc
+        rng = np.random.default_rng(seed)
+        self.ctx, self.T = ctx, T
+        self.w = {n: ctx.upload(t, synth.blocks(t, r, c, rng), r, c) for n, (t, r, c) in self.SHAPES.items()}
+        self.e = [ctx.upload(t, synth.blocks(t, 16 * r, c, rng), r, c, experts=16)
+                  for t, r, c in ((Q4_K, 256, 512), (Q4_K, 256, 512), (Q6_K, 512, 256))]
+        dev = lambda a: torch.from_numpy(np.ascontiguousarray(a, np.float32)).cuda()  # noqa: E731
+        self.x0, self.logits, self.norm = dev(rng.standard_normal((T, 512))), dev(rng.standard_normal((T, 16))), torch.ones(512, device="cuda")
+        self.c0 = torch.from_numpy(rng.standard_normal((2, 30 + T, 128)).astype(np.float16).view(np.int16)).cuda()
+        self.x, self.c, self.y = self.x0.clone(), self.c0.clone(), torch.empty_like(self.x0)
+        d = self.d = LayerDesc()
+        for n in self.w:
+            setattr(d, n, self.w[n].handle.value)
+        d.d_attn_norm = d.d_ffn_norm = self.norm.data_ptr()
+        d.embd, d.heads, d.kv_heads, d.head_dim, d.rope_dims = 512, 8, 2, 64, 64
+        d.rope_base, d.rope_freq_scale, d.eps = 10000.0, 1.0, 1e-6
+        torch.cuda.synchronize()
+
+    def run(self):
+        L, h = load(), self.ctx.handle
+        check(L.wl_layer_dev(h, ctypes.byref(self.d), _p(self.x), self.T, 30, _p(self.c[0]), _p(self.c[1])))
+        check(L.wl_moe_ffn_dev(h, _p(self.logits), 4, 1, self.e[0].handle, self.e[1].handle, self.e[2].handle, _p(self.x0),
+                               self.T, _p(self.y)))
+
+    def outputs(self):
+        self.ctx.sync()
+        return [t.clone() for t in (self.x.view(torch.int32), self.c, self.y.view(torch.int32))]
+
+    def reset(self):
+        self.x.copy_(self.x0)
+        self.c.copy_(self.c0)
+        self.y.fill_(float("nan"))
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("T", [12, 47, 200])
+def test_replayed_prompt_equals_eager_calls(T):
+    ctx = Context(0)
+    a, other = Prompt(ctx, T, T), Prompt(ctx, T, T + 1)
+    same = lambda got, want: all(torch.equal(g, w) for g, w in zip(got, want))  # noqa: E731
+    a.run()
+    want = a.outputs()
+    other.run()
+    other_want = other.outputs()
+    g = ctx.capture(a.run)
+    try:
+        for rep in range(3):
+            a.reset()
+            g.launch()
+            assert same(a.outputs(), want), rep
+            other.reset()
+            other.run()
+            assert same(other.outputs(), other_want), rep
+    finally:
+        g.free()
+        ctx.close()
